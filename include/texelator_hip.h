@@ -173,6 +173,18 @@ int tx_stream_read(const void *data, int64_t bytes, uint32_t *sink, void *stream
 /* Replaces texelator_free (texelator_cuda.cu:1538). Caller must ensure no work is pending. */
 int tx_free(uint64_t handle);
 
+/* BC4 encoding of a dense matrix on the GPU: the reference's activation-weighted endpoint search
+ * (texelator/encoder.py:35-157), which it runs as torch operations, in one launch.
+ *   weight   device [rows][K] of dtype (F32, BF16 or F16), K a multiple of 16
+ *   hdiag    device float32 [K]: the importance of each input column
+ *   lut      device float32 255 x 255 x 8 palette table in the probe layout (see tx_palette_probe)
+ *   blocks   device output [rows][K/16][8] bytes (the layout tx_pack_encoded_device takes)
+ *   scales   device output float32 [rows]: max |weight| of the row, at least 1e-12
+ * weight, hdiag and lut 16-byte aligned, blocks 8-byte aligned. The bytes are those of the torch
+ * operations of texelator_amd/encoder.py on the same device. Asynchronous on the stream. */
+int tx_encode_bc4(const void *weight, int dtype, int64_t rows, int64_t K, const float *hdiag, const float *lut,
+                  uint8_t *blocks, float *scales, int device, void *stream);
+
 /* Replaces texelator_palette_probe (texelator_cuda.cu:1551-1595): fills host_out with the
  * 255*255*8 float32 palette measured from the device decoder, index ((e1+127)*255+(e0+127))*8+s,
  * on the current device. Synchronous. */

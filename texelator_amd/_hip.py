@@ -129,6 +129,27 @@ def pack_encoded_device(blocks: torch.Tensor, scales: torch.Tensor, bias: torch.
     return handle
 
 
+def encode_bc4(weight: torch.Tensor, hdiag: torch.Tensor, lut: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """BC4 blocks uint8 ``[M, K/16*8]`` and row scales float32 ``[M]`` of a CUDA matrix ``weight`` [M, K]
+    (float32, bf16 or fp16) under column importances ``hdiag`` float32 [K] and the palette table
+    ``lut``, in one launch (``tx_encode_bc4``); all on one device, contiguous."""
+    codes = {torch.float32: _lib.TX_DTYPE_F32, **_DTYPE_CODE}
+    _require(weight.is_cuda and weight.dim() == 2 and weight.dtype in codes and weight.is_contiguous(),
+             "weight must be a contiguous CUDA float32, BF16 or FP16 matrix")
+    m, k = weight.shape
+    _require(all(t.device == weight.device and t.dtype == torch.float32 and t.is_contiguous() for t in (hdiag, lut)),
+             "hdiag and lut must be contiguous float32 on the weight's device")
+    _require(hdiag.numel() == k and lut.numel() == 255 * 255 * 8, "hdiag must hold K values, lut 255*255*8")
+    weight, hdiag, lut = _aligned(weight), _aligned(hdiag), _aligned(lut)
+    blocks = torch.empty((m, k // 16 * 8), dtype=torch.uint8, device=weight.device)
+    scales = torch.empty(m, dtype=torch.float32, device=weight.device)
+    check(_lib.load().tx_encode_bc4(ctypes.c_void_p(weight.data_ptr()), codes[weight.dtype], m, k,
+                                    ctypes.c_void_p(hdiag.data_ptr()), ctypes.c_void_p(lut.data_ptr()),
+                                    ctypes.c_void_p(blocks.data_ptr()), ctypes.c_void_p(scales.data_ptr()),
+                                    weight.device.index, _stream(weight.device)))
+    return blocks, scales
+
+
 def concat_rows(handles: list[int]) -> int:
     """A new handle with the rows of ``handles`` (one K) in order (``tx_concat_rows``); every handle
     but the last needs a multiple of 16 rows. The sources stay valid; free the result on its own."""

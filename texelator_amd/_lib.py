@@ -49,6 +49,7 @@ SIGNATURES = {
     "tx_free": (_I32, [_U64]),
     "tx_add_rmsnorm_bf16": (_I32, [_P, _P, _P, ctypes.c_float, _P, _P, _I64, _I64, _P]),
     "tx_concat_rows": (_I32, [ctypes.POINTER(_U64), _I32, ctypes.POINTER(_U64)]),
+    "tx_encode_bc4": (_I32, [_P, _I32, _I64, _I64, _P, _P, _P, _P, _I32, _P]),
     "tx_palette_probe": (_I32, [_P]),
     "tx_decode_dense": (_I32, [_U64, _I32, _P, _P]),
     "tx_kernel_info": (_I32, [_I32, ctypes.POINTER(_I64), _I32]),

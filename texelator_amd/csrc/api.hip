@@ -735,6 +735,24 @@ int tx_free(uint64_t value) {
   return TX_OK;
 }
 
+int tx_encode_bc4(const void *weight, int dtype, int64_t rows, int64_t K, const float *hdiag, const float *lut,
+                  uint8_t *blocks, float *scales, int device, void *stream) {
+  g_last_error.clear();
+  if (dtype != TX_DTYPE_F32 && dtype != TX_DTYPE_BF16 && dtype != TX_DTYPE_F16)
+    return fail(TX_ERR_INVALID, "encode_bc4: the weight must be FP32, BF16 or FP16");
+  if (K <= 0 || K % 16 || K > (1 << 30) || rows < 0 || rows > 0x7FFFFFFF)
+    return fail(TX_ERR_INVALID, "encode_bc4: K must be a positive multiple of 16");
+  if (!weight || !hdiag || !lut || !blocks || !scales) return fail(TX_ERR_INVALID, "encode_bc4: null pointer");
+  for (const void *ptr : {weight, static_cast<const void *>(hdiag), static_cast<const void *>(lut)})
+    if (reinterpret_cast<uintptr_t>(ptr) % 16) return fail(TX_ERR_INVALID, "encode_bc4: inputs must be 16-byte aligned");
+  if (reinterpret_cast<uintptr_t>(blocks) % 8) return fail(TX_ERR_INVALID, "encode_bc4: blocks must be 8-byte aligned");
+  if (rows == 0) return TX_OK;
+  DeviceGuard guard(device);
+  TX_HIP(tx::launch_encode(weight, dtype, rows, (int)K, hdiag, reinterpret_cast<const float4 *>(lut),
+                           reinterpret_cast<uint2 *>(blocks), scales, reinterpret_cast<hipStream_t>(stream)));
+  return TX_OK;
+}
+
 int tx_palette_probe(float *host_out) {
   g_last_error.clear();
   if (!host_out) return fail(TX_ERR_INVALID, "null output");

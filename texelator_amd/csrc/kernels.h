@@ -124,6 +124,11 @@ void prefill_candidate_shape(int candidate, int *tokens, int *rows, int *k);
 // Workgroups of a candidate one CU holds at once (occupancy query; 0 for an unknown id).
 int prefill_resident_per_cu(int candidate);
 
+// BC4 encoding of a dense matrix [rows][K] (K a multiple of 16; 16-byte aligned; dtype F32, BF16 or
+// F16): reference-layout blocks [rows][K/16] and row scales (encode.hip). hdiag: K importances.
+hipError_t launch_encode(const void *weight, int dtype, int64_t rows, int K, const float *hdiag, const float4 *lut,
+                         uint2 *blocks, float *scales, hipStream_t stream);
+
 hipError_t launch_palette_probe(float *out, hipStream_t stream);
 // Streaming read of bytes (a multiple of 16) with kStreamReadBlocks workgroups; sink receives at
 // most one word per workgroup (only for an input that XORs to a sentinel value).

@@ -4,7 +4,9 @@ Restates ``texelator/encoder.py`` of the reference. The arithmetic of the endpoi
 kept step for step (same float32 expressions and reductions) so that, on the CPU, the chosen
 endpoints and selectors are identical to the reference's for the same LUT; the code is
 organised differently (coefficient lookup tables, candidate loop over a fixed offset list).
-The encoder runs on whatever device ``lut`` lives on.
+The encoder runs on whatever device ``lut`` lives on. On a GPU a whole row chunk is one launch of the
+library's encoder kernel (``tx_encode_bc4``), which gives the bytes of the torch operations below on that
+GPU; those run on the CPU, and wherever :func:`endpoint_opt` is called with a scale of one's own.
 """
 from __future__ import annotations
 
@@ -141,6 +143,24 @@ def pack_blocks_tensor(endpoint0: torch.Tensor, endpoint1: torch.Tensor, indices
     return packed
 
 
+def _native_encode(lut: torch.Tensor, hdiag: torch.Tensor, k: int):
+    """The library's encoder for row chunks of K columns on ``lut``'s GPU: a function of a chunk (any
+    device, type or strides) giving ``(blocks, scales)`` device tensors; None where the torch
+    operations run (a CPU table, or a table or moments of another form)."""
+    if not (lut.is_cuda and lut.dtype == torch.float32 and lut.numel() == PALETTE_FLOATS and hdiag.numel() == k):
+        return None
+    from . import _hip
+
+    moments, table = hdiag.float().reshape(-1).contiguous(), lut.contiguous()
+
+    def encode(rows: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+        widened_there = rows.dtype in (torch.float32, torch.bfloat16, torch.float16)
+        rows = rows.detach().to(device=lut.device, dtype=rows.dtype if widened_there else torch.float32)
+        return _hip.encode_bc4(rows.contiguous(), moments, table)
+
+    return encode
+
+
 @torch.inference_mode()
 def encode_matrix_tensor(weight: torch.Tensor, hdiag: torch.Tensor, lut: torch.Tensor,
                          rows_per_chunk: int = 2048) -> tuple[torch.Tensor, torch.Tensor]:
@@ -150,13 +170,21 @@ def encode_matrix_tensor(weight: torch.Tensor, hdiag: torch.Tensor, lut: torch.T
     if k % 16:
         raise ValueError(f"unsupported K={k}; BC4 needs K % 16 == 0")
     hdiag = hdiag.to(lut.device)
+    native = _native_encode(lut, hdiag, k)
+    if native is not None and weight.device == lut.device and 0 < m <= 0x7FFFFFFF and rows_per_chunk > 0:
+        return native(weight)  # resident: nothing to stage and no scratch, so one launch
     blocks = torch.empty((m, k // 16 * 8), dtype=torch.uint8, device=lut.device)
     scales = torch.empty(m, dtype=torch.float32, device=lut.device)
     for start in range(0, m, rows_per_chunk):
-        rows = weight[start:start + rows_per_chunk].detach().float().to(lut.device)
-        row_scales = rows.abs().amax(1).clamp_min(1e-12)
-        e0, e1, idx = endpoint_opt(rows, hdiag, row_scales, lut)
-        blocks[start:start + rows.shape[0]] = pack_blocks_tensor(e0, e1, idx).reshape(rows.shape[0], -1)
+        rows = weight[start:start + rows_per_chunk]
+        if native is not None:
+            packed, row_scales = native(rows)
+        else:
+            rows = rows.detach().float().to(lut.device)
+            row_scales = rows.abs().amax(1).clamp_min(1e-12)
+            e0, e1, idx = endpoint_opt(rows, hdiag, row_scales, lut)
+            packed = pack_blocks_tensor(e0, e1, idx).reshape(rows.shape[0], -1)
+        blocks[start:start + rows.shape[0]] = packed
         scales[start:start + rows.shape[0]] = row_scales
     return blocks, scales
 
@@ -172,11 +200,17 @@ def encode_rows(weight: torch.Tensor, hdiag: torch.Tensor, lut: torch.Tensor,
     if k % 16:
         raise ValueError(f"unsupported K={k}; BC4 needs K % 16 == 0")
     hdiag = hdiag.to(lut.device)
+    native = _native_encode(lut, hdiag, k)
     for start in range(0, m, rows_per_chunk):
-        rows = weight[start:start + rows_per_chunk].detach().float().to(lut.device)
-        scales = rows.abs().amax(1).clamp_min(1e-12)
-        e0, e1, idx = endpoint_opt(rows, hdiag, scales, lut)
-        packed = pack_blocks(e0, e1, idx).reshape(rows.shape[0], -1)
+        rows = weight[start:start + rows_per_chunk]
+        if native is not None:
+            packed, scales = native(rows)
+            packed = packed.cpu().numpy()
+        else:
+            rows = rows.detach().float().to(lut.device)
+            scales = rows.abs().amax(1).clamp_min(1e-12)
+            e0, e1, idx = endpoint_opt(rows, hdiag, scales, lut)
+            packed = pack_blocks(e0, e1, idx).reshape(rows.shape[0], -1)
         yield packed, scales.cpu().numpy().astype("<f4", copy=False)
 
 
