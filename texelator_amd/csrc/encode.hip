@@ -9,7 +9,9 @@
 // encodes whole 16-value blocks in registers. As torch operations a 5120 x 5120 matrix took 26.1 ms:
 // about 1500 launches, each a pass over [blocks][16] arrays in memory. Here the weights are read once
 // from HBM (the second read of a row hits the caches) and only the blocks are written. What is left
-// is VALU work: nine candidate palettes of eight values against sixteen weights.
+// is VALU work: nine candidate palettes of eight values against sixteen weights, ~4000 instructions a
+// block; 174 us for that matrix, its issue floor being ~165. Five waves per SIMD (96 registers, 124 bytes
+// spilled in the least squares) hide the palette gathers better than three without spills (238 us).
 #include "bc4_device.h"
 #include "kernels.h"
 
@@ -90,23 +92,20 @@ __device__ __forceinline__ void load16(const void *w, size_t first, float (&v)[1
 // The larger of two maxima, NaN if either is (torch.amax).
 __device__ __forceinline__ float max_nan(float a, float b) { return a != a ? a : (b > a || b != b ? b : a); }
 
-// Weights (a, b, c) of q = a*u + b*z + c for a selector in 8-value mode (c = 0) or 6-value mode.
-__device__ __forceinline__ void coefficients(uint32_t s, bool eight, float &a, float &b, float &c) {
-  constexpr float a8[8] = {1.0f, 0.0f, (float)(6.0 / 7), (float)(5.0 / 7), (float)(4.0 / 7), (float)(3.0 / 7), (float)(2.0 / 7), (float)(1.0 / 7)};
-  constexpr float b8[8] = {0.0f, 1.0f, (float)(1.0 / 7), (float)(2.0 / 7), (float)(3.0 / 7), (float)(4.0 / 7), (float)(5.0 / 7), (float)(6.0 / 7)};
-  constexpr float a6[8] = {1.0f, 0.0f, (float)(4.0 / 5), (float)(3.0 / 5), (float)(2.0 / 5), (float)(1.0 / 5), 0.0f, 0.0f};
-  constexpr float b6[8] = {0.0f, 1.0f, (float)(1.0 / 5), (float)(2.0 / 5), (float)(3.0 / 5), (float)(4.0 / 5), 0.0f, 0.0f};
-  a = b = 0.f;
-#pragma unroll
-  for (uint32_t i = 0; i < 8; ++i) {
-    a = s == i ? (eight ? a8[i] : a6[i]) : a;
-    b = s == i ? (eight ? b8[i] : b6[i]) : b;
-  }
-  c = eight || s < 6 ? 0.f : (s == 6 ? -1.f : 1.f);
-}
+// Weights of q = a*u + b*z + c by mode (6 values, 8 values) and selector, as {a, b, c, 0}: a copy in
+// LDS, read by the selector (selecting among constants took 22 VALU instructions a weight).
+__constant__ const float kCoefficients[2][8][4] = {
+    {{1.f, 0.f, 0.f, 0.f}, {0.f, 1.f, 0.f, 0.f}, {(float)(4.0 / 5), (float)(1.0 / 5), 0.f, 0.f},
+     {(float)(3.0 / 5), (float)(2.0 / 5), 0.f, 0.f}, {(float)(2.0 / 5), (float)(3.0 / 5), 0.f, 0.f},
+     {(float)(1.0 / 5), (float)(4.0 / 5), 0.f, 0.f}, {0.f, 0.f, -1.f, 0.f}, {0.f, 0.f, 1.f, 0.f}},
+    {{1.f, 0.f, 0.f, 0.f}, {0.f, 1.f, 0.f, 0.f}, {(float)(6.0 / 7), (float)(1.0 / 7), 0.f, 0.f},
+     {(float)(5.0 / 7), (float)(2.0 / 7), 0.f, 0.f}, {(float)(4.0 / 7), (float)(3.0 / 7), 0.f, 0.f},
+     {(float)(3.0 / 7), (float)(4.0 / 7), 0.f, 0.f}, {(float)(2.0 / 7), (float)(5.0 / 7), 0.f, 0.f},
+     {(float)(1.0 / 7), (float)(6.0 / 7), 0.f, 0.f}}};
 
 // One block: values v (weight / scale clamped to [-1, 1]) and importances h -> its 8 bytes.
-__device__ __forceinline__ uint2 encode_one(const float (&v)[16], const float (&h)[16], const float4 *lut) {
+__device__ __forceinline__ uint2 encode_one(const float (&v)[16], const float (&h)[16], const float4 *lut,
+                                            const float4 (&coefficients)[2][8]) {
   // 1. start: endpoints at the largest and smallest value, selectors nearest
   float hi = v[0], lo = v[0];
 #pragma unroll
@@ -125,12 +124,11 @@ __device__ __forceinline__ uint2 encode_one(const float (&v)[16], const float (&
     float aa[16], bb[16], ab[16], ay[16], by[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      float a, b, c;
-      coefficients(nearest_index(v[i], row), eight, a, b, c);
-      const float ha = h[i] * a, hb = h[i] * b, target = v[i] - c;
-      aa[i] = ha * a;
-      bb[i] = hb * b;
-      ab[i] = ha * b;
+      const float4 w = coefficients[eight][nearest_index(v[i], row)];
+      const float ha = h[i] * w.x, hb = h[i] * w.y, target = v[i] - w.z;
+      aa[i] = ha * w.x;
+      bb[i] = hb * w.y;
+      ab[i] = ha * w.y;
       ay[i] = ha * target;
       by[i] = hb * target;
     }
@@ -179,11 +177,13 @@ __device__ __forceinline__ uint2 encode_one(const float (&v)[16], const float (&
 }
 
 template <int DT>
-__global__ __launch_bounds__(kEncodeMaxThreads) void encode_rows_kernel(const void *weight, int K, const float *hdiag,
+__global__ __launch_bounds__(kEncodeMaxThreads, 5) void encode_rows_kernel(const void *weight, int K, const float *hdiag,
                                                                         const float4 *lut, uint2 *blocks, float *scales) {
   __shared__ float wave_max_[kEncodeMaxThreads / 64];
+  __shared__ float4 coefficients[2][8];
   const size_t row = blockIdx.x;
   const int nblk = K / 16, tid = threadIdx.x, threads = blockDim.x;
+  if (tid < 64) reinterpret_cast<float *>(coefficients)[tid] = reinterpret_cast<const float *>(kCoefficients)[tid];
   float v[16];
   float m = 0.f;
   for (int b = tid; b < nblk; b += threads) {
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(kEncodeMaxThreads) void encode_rows_kernel(const vo
     load16<kF32>(hdiag, (size_t)b * 16, h);
 #pragma unroll
     for (int i = 0; i < 16; ++i) v[i] = clamp_nan(v[i] / scale, -1.f, 1.f);
-    blocks[row * nblk + b] = encode_one(v, h, lut);
+    blocks[row * nblk + b] = encode_one(v, h, lut, coefficients);
   }
 }
 
