@@ -617,218 +617,6 @@ __global__ __launch_bounds__(128) void decode_attention_combine_kernel(const flo
   out[(size_t)head * kHeadDim + dd] = to_bf(((acc[0] + acc[1]) + (acc[2] + acc[3])) / total);
 }
 
-// Causal self-attention of a prompt: query tokens 0..T-1 against keys 0..T-1 (the prompt's own
-// cache rows), grouped-query, head_dim 128. Block (query block of 64, head), heaviest query blocks
-// first, HALVES sets of 4 waves: the waves of half hf take the key blocks kb = hf, hf + HALVES, ...
-// up to the diagonal (with two halves a query block's chain of dependent key blocks is half as
-// long, for grids too small to fill the GPU); wave w of a half owns queries 64*qb + 16w .. +15.
-// For each of its key blocks of 64 keys: the block's keys (padded rows) and values (transposed:
-// lane l loads dimensions 2l, 2l+1 of eight consecutive keys, one coalesced 256-byte key row per
-// load, and writes them as two 8-key runs) go to the half's LDS tiles, staged through registers
-// one of the half's blocks ahead; scores S = q k^T on the matrix cores (bf16 products, fp32 sums),
-// scaled by scale*log2(e) and masked causally on the diagonal block; an online softmax in fp32 with
-// exp2 (running max m and sum l per query; row reductions over the 16 lanes of a DPP row), the
-// output rescaled by exp2(m_old - m_new); the probabilities rounded to bf16 (their rounded values
-// summed into l) and multiplied by the values on the matrix cores (fp32 sums). With two halves
-// their (m, l, O) meet in LDS at the end: O = O0 exp2(m0 - M) + O1 exp2(m1 - M) and likewise l,
-// M = max(m0, m1). out = bf16(O / l). Values of keys past the prompt are zeroed, so stale cache
-// rows never reach the sums.
-constexpr int kPromptQueries = 64;
-
-
-constexpr int kKeyTileBytes = kChunk * kKeyStrideU4 * 16;   // keys [key][128] bf16, padded rows
-constexpr int kValueTileBytes = kHeadDim * kChunk * 2;      // values [dim][key] bf16 (vt_index)
-constexpr int kMergeFloats = 4 + 4 + 32;                    // m[4], l[4], O[8][4] of a lane
-
-template <int HALVES>
-__global__ __launch_bounds__(256 * HALVES, HALVES == 1 ? 2 : 1) void prefill_attention_kernel(
-    const uint16_t *q, int64_t q_stride, const uint16_t *k_cache, const uint16_t *v_cache, int tokens, int group,
-    int64_t max_ctx, float scale, uint16_t *out, int64_t out_stride) {
-  // Per half: a key tile and a value tile; after the K loop the same bytes carry half 1's (m, l, O).
-  __shared__ __align__(16) char tiles[HALVES * (kKeyTileBytes + kValueTileBytes)];
-  __shared__ __align__(16) uint16_t ps[4 * HALVES][16][kPRow];  // per wave: probabilities [query][key] bf16
-  static_assert(HALVES == 1 || 4 * kMergeFloats * 64 * 4 <= HALVES * (kKeyTileBytes + kValueTileBytes), "merge area");
-  const int qb = (int)gridDim.x - 1 - (int)blockIdx.x, head = blockIdx.y, kv = head / group;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  // half, wave within it, thread within it (compile-time constants with one half)
-  const int hf = HALVES == 1 ? 0 : wave >> 2, wq = HALVES == 1 ? wave : wave & 3, ht = HALVES == 1 ? tid : tid & 255;
-  uint4 *ks = reinterpret_cast<uint4 *>(tiles + hf * (kKeyTileBytes + kValueTileBytes));
-  uint16_t *vt = reinterpret_cast<uint16_t *>(tiles + hf * (kKeyTileBytes + kValueTileBytes) + kKeyTileBytes);
-  const int n = lane & 15, q4 = lane >> 4;
-  const int q0 = qb * kPromptQueries + 16 * wq;  // this wave's first query
-  const float sl2 = scale * 1.44269504088896340736f;  // scores in log2 units
-  // q as MFMA A operands: row n = query q0 + n (clamped into the prompt), dimensions 32 st + 8 q4 ..
-  dwordx4 qa[4];
-  {
-    const uint16_t *qr = q + (size_t)min(q0 + n, tokens - 1) * q_stride + (size_t)head * kHeadDim;
-#pragma unroll
-    for (int st = 0; st < 4; ++st) qa[st] = *reinterpret_cast<const dwordx4 *>(qr + 32 * st + 8 * q4);
-  }
-  // (32-bit byte offsets from the head's base: a head's cache is well under 4 GiB)
-  const char *kg = reinterpret_cast<const char *>(k_cache + (size_t)kv * max_ctx * kHeadDim);
-  const char *vg = reinterpret_cast<const char *>(v_cache + (size_t)kv * max_ctx * kHeadDim);
-  struct Block {
-    dwordx4 k[4];      // keys: 16-byte pieces idx = u * 256 + ht (key idx / 16, dimensions 8 (idx % 16) ..)
-    uint32_t v[16];    // values: dimensions 2 lane, 2 lane + 1 of keys 8 (2 wq + j / 8) + j % 8
-  };
-  // Blocks past the diagonal are never loaded (the clamp keeps every address inside the cache).
-  auto load_block = [&](Block &b, int kb) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int idx = u * 256 + ht;
-      const uint32_t row = (uint32_t)min((int64_t)(kb * kChunk + idx / kRowU4), max_ctx - 1);
-      b.k[u] = *reinterpret_cast<const dwordx4 *>(kg + (row * kRowU4 + idx % kRowU4) * 16u);
-    }
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const uint32_t row = (uint32_t)min((int64_t)(kb * kChunk + 16 * wq + j), max_ctx - 1);
-      b.v[j] = *reinterpret_cast<const uint32_t *>(vg + (row * kHeadDim + 2 * lane) * 2u);
-    }
-  };
-  float m[4], l[4];  // running max (log2 units) and sum of the lane's rows, queries q0 + 4 q4 + r
-  f32x4_t o[8];      // o[dt][r] = O[query q0 + 4 q4 + r][dimension 16 dt + n]
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    m[r] = -INFINITY;
-    l[r] = 0.f;
-  }
-#pragma unroll
-  for (int dt = 0; dt < 8; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  // One turn: the half's block kb = HALVES * it + hf from `blk`, whose registers then take the
-  // half's next block (loaded while this one is multiplied). Every half runs every turn (the
-  // barriers are workgroup-wide); a half whose blocks have run out idles through it.
-  auto turn = [&](int it, Block &blk) __attribute__((always_inline)) {
-    const int kb = HALVES * it + hf;
-    const bool active = HALVES == 1 || kb <= qb;  // one half runs every block up to the diagonal
-    __syncthreads();  // the previous block's tiles are no longer read
-    if (active) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int idx = u * 256 + ht;
-        reinterpret_cast<dwordx4 *>(ks)[(idx / kRowU4) * kKeyStrideU4 + idx % kRowU4] = blk.k[u];
-      }
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        const int key0 = 16 * wq + 8 * half;  // eight keys of this thread's run
-        uint32_t w[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = kb * kChunk + key0 + j < tokens ? blk.v[8 * half + j] : 0u;
-        const uint4 lo = make_uint4(__builtin_amdgcn_perm(w[1], w[0], 0x05040100u), __builtin_amdgcn_perm(w[3], w[2], 0x05040100u),
-                                    __builtin_amdgcn_perm(w[5], w[4], 0x05040100u), __builtin_amdgcn_perm(w[7], w[6], 0x05040100u));
-        const uint4 hi = make_uint4(__builtin_amdgcn_perm(w[1], w[0], 0x07060302u), __builtin_amdgcn_perm(w[3], w[2], 0x07060302u),
-                                    __builtin_amdgcn_perm(w[5], w[4], 0x07060302u), __builtin_amdgcn_perm(w[7], w[6], 0x07060302u));
-        *reinterpret_cast<uint4 *>(&vt[vt_index(2 * lane, key0)]) = lo;
-        *reinterpret_cast<uint4 *>(&vt[vt_index(2 * lane + 1, key0)]) = hi;
-      }
-    }
-    __syncthreads();
-    if (active && kb + HALVES <= qb) load_block(blk, kb + HALVES);  // in flight while this block is multiplied
-    float alpha[4];
-    if (active) {
-      // scores of sub-tile s (keys 16 s .. 16 s + 15 of the block): sc[s][r] = S[query q0+4q4+r][key 16s+n]
-      f32x4_t sc[4];
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4) {
-        const uint4 *krow = ks + (16 * s4 + n) * kKeyStrideU4;
-        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          const uint4 b = krow[4 * st + q4];
-          acc = mfma_bf16(qa[st], dwordx4{b.x, b.y, b.z, b.w}, acc);
-        }
-        sc[s4] = acc;
-      }
-      const bool diagonal = kb == qb;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float mx = -INFINITY;
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-          const int key = kb * kChunk + 16 * s4 + n, query = q0 + 4 * q4 + r;
-          float v = sc[s4][r] * sl2;
-          if (diagonal && (key > query || key >= tokens)) v = -INFINITY;
-          sc[s4][r] = v;
-          mx = fmaxf(mx, v);
-        }
-        // Every row has an unmasked key in every block up to the diagonal (key 64 kb <= query), so
-        // the running max is finite from a half's first block on.
-        const float mnew = fmaxf(m[r], row16_max(mx));
-        alpha[r] = __builtin_amdgcn_exp2f(m[r] - mnew);
-        m[r] = mnew;
-        float rs = 0.f;
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-          const uint16_t pb = to_bf(__builtin_amdgcn_exp2f(sc[s4][r] - mnew));
-          ps[wave][4 * q4 + r][16 * s4 + n] = pb;
-          rs += bf(pb);
-        }
-        l[r] = l[r] * alpha[r] + row16_sum(rs);
-      }
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[dt][r] *= alpha[r];
-    }
-    __syncthreads();  // the probabilities are in LDS
-    if (active) {
-      // O += P V: A = the probabilities (row n, keys 32 kst + 8 q4 ..), B = the transposed values
-#pragma unroll
-      for (int kst = 0; kst < kChunk / 32; ++kst) {
-        const uint4 a = *reinterpret_cast<const uint4 *>(&ps[wave][n][32 * kst + 8 * q4]);
-        const dwordx4 av = {a.x, a.y, a.z, a.w};
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) {
-          const uint4 b = *reinterpret_cast<const uint4 *>(&vt[vt_index(16 * dt + n, 32 * kst + 8 * q4)]);
-          o[dt] = mfma_bf16(av, dwordx4{b.x, b.y, b.z, b.w}, o[dt]);
-        }
-      }
-    }
-  };
-  const int turns = (qb + HALVES) / HALVES;
-  Block cur;
-  if (hf <= qb) load_block(cur, hf);
-  for (int it = 0; it < turns; ++it) turn(it, cur);
-
-  if constexpr (HALVES == 2) {
-    // Half 1 hands its (m, l, O) to half 0 through the tile bytes ([wq][item][lane] floats); a half
-    // that processed no block hands m = -inf, l = 0, O = 0, which the merge weighs by zero.
-    __syncthreads();  // every tile read is done
-    float *mg = reinterpret_cast<float *>(tiles) + wq * kMergeFloats * 64 + lane;
-    if (hf == 1) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        mg[r * 64] = m[r];
-        mg[(4 + r) * 64] = l[r];
-      }
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) mg[(8 + 4 * dt + r) * 64] = o[dt][r];
-    }
-    __syncthreads();
-    if (hf == 1) return;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float m1 = mg[r * 64], l1 = mg[(4 + r) * 64];
-      const float mm = fmaxf(m[r], m1);  // m[r] is finite: half 0 processed key block 0
-      const float a0 = __builtin_amdgcn_exp2f(m[r] - mm), a1 = __builtin_amdgcn_exp2f(m1 - mm);
-      l[r] = l[r] * a0 + l1 * a1;
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt) o[dt][r] = o[dt][r] * a0 + mg[(8 + 4 * dt + r) * 64] * a1;
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int query = q0 + 4 * q4 + r;
-    if (query >= tokens) continue;
-    const float inv = 1.0f / l[r];
-    uint16_t *dst = out + (size_t)query * out_stride + (size_t)head * kHeadDim + n;
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) dst[16 * dt] = to_bf(o[dt][r] * inv);
-  }
-}
-
 // Greedy next token of a dense bf16 lm_head W [vocab][hidden] for one hidden state x [hidden]:
 // token = the first v with the largest bf16(sum_k x[k] W[v][k]) (fp32 sums), as argmax over the
 // bf16 logits of a linear layer picks it. First pass: workgroup b takes a contiguous range of
@@ -1094,28 +882,6 @@ hipError_t launch_attention(const AttnInput &in, uint16_t *k_cache, uint16_t *v_
   return hipGetLastError();
 }
 }  // namespace
-
-bool prefill_attention_supported(int heads, int kv_heads, int head_dim) {
-  return head_dim == kHeadDim && kv_heads > 0 && heads % kv_heads == 0;
-}
-
-hipError_t launch_prefill_attention(const uint16_t *q, int64_t q_stride, const uint16_t *k_cache,
-                                    const uint16_t *v_cache, int64_t tokens, int heads, int kv_heads, int64_t max_ctx,
-                                    float scale, uint16_t *out, int64_t out_stride, hipStream_t stream) {
-  const dim3 grid((unsigned)((tokens + kPromptQueries - 1) / kPromptQueries), (unsigned)heads);
-  // Two halves per query block where the 4-wave blocks would not give every CU one (16 heads at
-  // 512 tokens: 18.8 -> 16.3 us); otherwise 4-wave blocks, two per CU (40 heads: 25.5 vs 32.6 us).
-  int device = 0, cus = 0;
-  if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
-    return hipGetLastError();
-  if ((int64_t)grid.x * grid.y <= cus)
-    hipLaunchKernelGGL(prefill_attention_kernel<2>, grid, dim3(512), 0, stream, q, q_stride, k_cache, v_cache, (int)tokens,
-                       heads / kv_heads, max_ctx, scale, out, out_stride);
-  else
-    hipLaunchKernelGGL(prefill_attention_kernel<1>, grid, dim3(256), 0, stream, q, q_stride, k_cache, v_cache, (int)tokens,
-                       heads / kv_heads, max_ctx, scale, out, out_stride);
-  return hipGetLastError();
-}
 
 hipError_t launch_decode_attention(const uint16_t *q, const uint16_t *k_cache, const uint16_t *v_cache,
                                    const int64_t *position, int64_t length, int heads, int kv_heads, int64_t max_ctx,
