@@ -68,7 +68,8 @@ int tx_concat_rows(const uint64_t *handles, int count, uint64_t *handle_out);
  *   workspace device scratch of at least tx_workspace_bytes(handle, tokens) bytes, 16-byte
  *             aligned (may be NULL when that is 0), stream-ordered: the prefill path's split-K
  *             partials or backend 1's dense rows (required), or a one-token GEMV's split-K partials (optional: with NULL the
- *             handle's own buffer is used, so two such calls on one handle must not overlap)
+ *             handle's own buffer is used, so two such calls on one handle must not overlap), or
+ *             the batched GEMV's for a few tokens (optional: see tx_linear_workspace_bytes)
  * tokens >= prefill threshold (and tokens > 1) uses the prefill GEMM candidate set by
  * tx_set_prefill_backend; otherwise the decode GEMV with the configured lookahead.
  * The reference allocates its prefill scratch inside the call (texelator_cuda.cu:942-957); here
@@ -124,6 +125,12 @@ int tx_noalloc_scratch_bytes(int64_t *bytes);
  * its splits: 2 to 4 splits, row groups spreading evenly over the CUs, arithmetic palette). No
  * reference counterpart (see tx_linear). */
 int tx_workspace_bytes(uint64_t handle, int64_t tokens, int64_t *bytes);
+
+/* Workspace bytes tx_linear itself can use for `tokens` tokens: tx_workspace_bytes for one token and at or
+ * above the prefill threshold; for several tokens below it the K-split partials of the batched GEMV
+ * (2 to 16 tokens; 0 where it does not run). There the workspace is optional: without one of this size
+ * tx_linear runs that call unsplit, slower, with sums in another order. */
+int tx_linear_workspace_bytes(uint64_t handle, int64_t tokens, int64_t *bytes);
 
 /* Decode GEMV with float32 output and no bias, for parity checks (no reference counterpart:
  * the reference only returns 16-bit outputs). x: device bf16 [tokens][K]; y: device f32. One-token

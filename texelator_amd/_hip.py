@@ -55,11 +55,16 @@ def workspace_bytes(handle: int, tokens: int) -> int:
     return int(out.value)
 
 
-def _workspace(handle: int, tokens: int, device: torch.device):
+def _workspace(handle: int, tokens: int, device: torch.device, linear: bool = False):
     """Stream-ordered scratch from the caching allocator (None when the shape needs none): the
-    prefill split-K partials, or a one-token GEMV's, so that calls on one handle from several
-    streams never share the handle's own buffer."""
-    nbytes = workspace_bytes(handle, tokens) if tokens >= 1 else 0
+    prefill split-K partials, or (``linear``) those of a GEMV of one or a few tokens, so that calls on
+    one handle from several streams never share the handle's own buffer."""
+    nbytes = 0
+    if tokens >= 1:
+        out = ctypes.c_int64(0)
+        query = _lib.load().tx_linear_workspace_bytes if linear else _lib.load().tx_workspace_bytes
+        check(query(handle, tokens, ctypes.byref(out)))
+        nbytes = out.value
     if nbytes == 0:
         return None, ctypes.c_void_p(None), 0
     ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
@@ -174,7 +179,7 @@ def linear(handle: int, x: torch.Tensor) -> torch.Tensor:
     y = torch.empty(out_shape, dtype=x.dtype, device=x.device)
     x = _aligned(x)
     tokens = x.numel() // k
-    ws, ws_ptr, ws_bytes = _workspace(handle, tokens, x.device)
+    ws, ws_ptr, ws_bytes = _workspace(handle, tokens, x.device, linear=True)
     check(_lib.load().tx_linear(handle, ctypes.c_void_p(x.data_ptr()), _DTYPE_CODE[x.dtype], x.numel(),
                                 x.size(-1), x.device.index, ctypes.c_void_p(y.data_ptr()), ws_ptr, ws_bytes,
                                 _stream(x.device)))

@@ -34,6 +34,7 @@ SIGNATURES = {
     "tx_pack_encoded_device": (_I32, [_P, _I64, _P, _I64, _P, _I32, _I32, ctypes.POINTER(_U64)]),
     "tx_linear": (_I32, [_U64, _P, _I32, _I64, _I64, _I32, _P, _P, _I64, _P]),
     "tx_workspace_bytes": (_I32, [_U64, _I64, ctypes.POINTER(_I64)]),
+    "tx_linear_workspace_bytes": (_I32, [_U64, _I64, ctypes.POINTER(_I64)]),
     "tx_linear_noalloc": (_I32, [_U64, _P, _I32, _I64, _I64, _I32, _P, _P]),
     "tx_noalloc_scratch_bytes": (_I32, [ctypes.POINTER(_I64)]),
     "tx_quantize_activation_fp4": (_I32, [_P, _I32, _I64, _I64, _P, _P, _I32, _P]),

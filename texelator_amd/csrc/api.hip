@@ -235,6 +235,16 @@ int64_t gemv_partials_bytes(const Handle *h, int64_t tokens) {
   return (int64_t)h->gemv_splits * h->Mp * (int64_t)sizeof(float);
 }
 
+// Partials of a call of several tokens below the prefill threshold: bytes, 0 where it runs unsplit
+// without any (more than 16 tokens, or partials past kBatchPartialsLimit).
+constexpr int64_t kBatchPartialsLimit = (int64_t)kScratchBytes;
+int64_t batch_partials_bytes(const Handle *h, int64_t tokens) {
+  const int64_t bytes = (int64_t)tx::gemv_batch_splits(h->RG, h->CG, h->K, tokens, h->cus) * tokens * h->Mp * (int64_t)sizeof(float);
+  return bytes <= kBatchPartialsLimit ? bytes : 0;
+}
+
+// partials: for one token (unless its GEMV needs none) gemv_partials_bytes of scratch; for several,
+// batch_partials_bytes of it or nullptr (then the unsplit kernel runs).
 int run_gemv(Handle *h, const void *x, bool f16, int64_t tokens, void *y, bool f32_out, hipStream_t stream,
              float *partials) {
   if (tokens > 65535) return fail(TX_ERR_INVALID, "token grid exceeds the HIP grid.z limit");
@@ -252,9 +262,14 @@ int run_gemv(Handle *h, const void *x, bool f16, int64_t tokens, void *y, bool f
   p.RG = h->RG;
   p.CG = h->CG;
   p.tokens = (int)tokens;
+  p.partials = partials;
+  if (tokens > 1 && !f32_out && partials && batch_partials_bytes(h, tokens) > 0) {
+    p.ks = tx::gemv_batch_splits(h->RG, h->CG, h->K, tokens, h->cus);
+    TX_HIP(tx::launch_gemv_batch(p, stream));
+    return TX_OK;
+  }
   // One token: K splits reduced by a second kernel. Several tokens: one pass per 16 tokens.
   p.ks = tokens == 1 ? h->gemv_splits : 1;
-  p.partials = partials;
   p.fused = tokens == 1 && one_token_fused(h) ? 1 : 0;
   TX_HIP(tx::launch_gemv(p, h->lookahead, f32_out, stream));
   return TX_OK;
@@ -511,9 +526,9 @@ int tx_linear(uint64_t value, const void *x, int x_dtype, int64_t x_numel, int64
   if (h->bias && h->bias_dtype != x_dtype) return fail(TX_ERR_INVALID, "input and bias dtypes must match");
   // A caller workspace large enough for the one-token split-K partials keeps concurrent calls on
   // one handle apart; without one the handle's own buffer is used (calls must then not overlap).
-  const int64_t need = gemv_partials_bytes(h, tokens);
+  const int64_t need = tokens == 1 ? gemv_partials_bytes(h, tokens) : batch_partials_bytes(h, tokens);
   const bool own = need > 0 && workspace && workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0;
-  return run_gemv(h, x, f16, tokens, y, false, s, own ? static_cast<float *>(workspace) : h->partials);
+  return run_gemv(h, x, f16, tokens, y, false, s, own ? static_cast<float *>(workspace) : tokens == 1 ? h->partials : nullptr);
 }
 
 int tx_linear_add_bias(uint64_t value, const void *x, const void *bias, void *y, void *stream) {
@@ -668,6 +683,16 @@ int tx_workspace_bytes(uint64_t value, int64_t tokens, int64_t *bytes) {
   if (!bytes) return fail(TX_ERR_INVALID, "null output");
   if (tokens > 1 && tokens >= h->prefill_threshold) *bytes = prefill_call_bytes(h, tokens);
   else *bytes = tokens > 1 ? prefill_workspace_bytes(h, tokens) : gemv_partials_bytes(h, tokens);
+  return TX_OK;
+}
+
+int tx_linear_workspace_bytes(uint64_t value, int64_t tokens, int64_t *bytes) {
+  g_last_error.clear();
+  Handle *h = as_handle(value);
+  if (!h) return fail(TX_ERR_INVALID, "null Texelator handle");
+  if (!bytes) return fail(TX_ERR_INVALID, "null output");
+  if (tokens > 1 && tokens >= h->prefill_threshold) *bytes = prefill_call_bytes(h, tokens);
+  else *bytes = tokens > 1 ? batch_partials_bytes(h, tokens) : gemv_partials_bytes(h, tokens);
   return TX_OK;
 }
 

@@ -15,6 +15,8 @@
 //     spread evenly over the CUs, one workgroup instead runs every split of its row group and sums
 //     them in the same order (gemv_fused_kernel: the same bits, one launch).
 // Single-token calls stage x in LDS; multi-token calls read x through the cache hierarchy.
+#include <algorithm>
+
 #include "bc4_device.h"
 #include "elementwise.h"
 #include "kernels.h"
@@ -525,6 +527,91 @@ __global__ __launch_bounds__(kThreads, LUT || XSRC != kXRead ? 4 : TX_GEMV_WAVES
   }
 }
 
+// Several tokens (2 to 16) through one pass of the weights where K is long (gemv_batch_splits), K split so that the chip is full whatever the
+// matrix's shape: a workgroup of eight waves takes eight row groups (one per wave) x one K range, with
+// the range's activations of all tokens in LDS, and writes fp32 partials [split][token][Mp] that
+// splitk_reduce_kernel sums in split order. Each wave streams the whole range of its own row group, so
+// nothing crosses waves and the K loop has no barrier.
+//   * What bounds it is the decode, as in the one-token kernel; gemv_kernel<MULTI> instead read every
+//     tile's activations through the cache hierarchy (4 KiB per 1 KiB of weights, in the decode's way) and
+//     could not split K, so a matrix of few rows left most of the chip idle. Main kernel and reduce: 5120 x
+//     27648 at 8 tokens 46.6 -> 25.7 us, 27648 x 5120 at 8 31.6 -> 24.4 us, at 15 46.0 -> 28.7 us.
+//   * LDS: column c of the range, token t, chunk q (8 k-values) at 16-byte slot 16 (R c + t) + (q ^ (t % 16)), R = tokens
+//     rounded up to 4 (whole 1 KiB direct loads): the sixteen tokens an MFMA operand read serves fall on
+//     distinct banks. Tokens past the last and columns past K read as zeros (offsets past the descriptor).
+constexpr int kBatchWaves = 8;
+constexpr int kBatchLdsBytes = 56 << 10;  // activations of a workgroup: two workgroups a CU at the most tokens
+
+template <bool F16, bool LUT>
+__global__ __launch_bounds__(64 * kBatchWaves, LUT ? 4 : 6) void gemv_batch_kernel(GemvParams p) {
+  extern __shared__ uint4 xs[];
+  __shared__ __attribute__((aligned(16))) PaletteTableStorage tables;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int split = blockIdx.y;
+  const int c_begin = (int)((uint32_t)split * (uint32_t)p.CG / (uint32_t)p.ks);
+  const int nc = (int)((uint32_t)(split + 1) * (uint32_t)p.CG / (uint32_t)p.ks) - c_begin;
+  const int g = (int)blockIdx.x * kBatchWaves + wave;
+  const bool active = g < p.RG;
+  const int gc = active ? g : p.RG - 1;  // a wave past the last row group repeats it and stores nothing
+  const int64_t first_tile = (int64_t)gc * p.CG + c_begin;
+  const TileStream stream(p.tiles + first_tile * 64, ((int64_t)p.RG * p.CG - first_tile) * kTileBytes, lane);
+  constexpr int LA = 2, R = LA + 1;
+  uint4 ring[R];
+#pragma unroll
+  for (int u = 0; u < LA; ++u) ring[u] = stream.load(u, nc, 1);
+  const int i = lane & 15, kg = lane >> 4;
+  const float scale = p.scales[gc * kTileRows + i];
+
+  const int rows4 = (p.tokens + 3) / 4;  // 1 KiB loads (four tokens) per column
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void *>(p.x), (short)0, (int)((int64_t)p.tokens * p.K * 2), 0x00020000);
+  for (int q = wave; q < nc * rows4; q += kBatchWaves) {
+    const int c = q / rows4, t = (q - c * rows4) * 4 + kg;
+    const int k = (c_begin + c) * kTileK + 8 * (i ^ t);
+    const uint32_t off = t < p.tokens && k < p.K ? (uint32_t)(t * p.K + k) * 2u : 0x7FFFFFF0u;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void *)(xs + q * 64), 16, off, 0, 0, 0);
+  }
+  if constexpr (!LUT) copy_seed_tables(tables, wave, lane, kBatchWaves);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the activations and tables have landed
+  __syncthreads();
+
+  const uint32_t pm = pm_scale_pair<F16>(scale);
+  const int tl = min(i, 4 * rows4 - 1);  // token column of this lane (columns past the tokens are not stored)
+  const uint4 *xt = xs + tl * 16;
+  f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+  auto load_xf = [&](XFrag &xf, int j) {
+    const uint4 *xv = xt + j * rows4 * 64;
+    xf.x0 = xv[(4 * kg) ^ tl];
+    xf.x1 = xv[(4 * kg + 1) ^ tl];
+    xf.x2 = xv[(4 * kg + 2) ^ tl];
+    xf.x3 = xv[(4 * kg + 3) ^ tl];
+  };
+  auto tile = [&](int j, const uint4 &cur) {
+    XFrag xf;
+    load_xf(xf, j);
+    if constexpr (LUT) tile_mfma_lut<F16>(cur, tile_rows(p.lut, cur), xf, scale, acc0, acc1);
+    else tile_mfma<F16>(cur, xf, scale, pm, tables, acc0, acc1);
+  };
+  int j0 = 0;
+  for (; j0 + R <= nc; j0 += R) {
+    progress_priority(nc - j0, nc);
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      ring[(u + LA) % R] = stream.load(j0 + u + LA, nc, 1);
+      tile(j0 + u, ring[u]);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < LA; ++u)
+    if (j0 + u < nc) tile(j0 + u, ring[u]);
+
+  // acc[r] = partial y[token i][row 4kg + r]
+  const f32x4 acc = acc0 + acc1;
+  if (active && i < p.tokens)
+    *reinterpret_cast<f32x4 *>(p.partials + ((size_t)split * p.tokens + i) * p.Mp + g * kTileRows + 4 * kg) = acc;
+}
+
 // One token, every K split in one workgroup: 4 * ks waves (ks <= kFusedMaxSplits) for one 16-row
 // group, wave w doing exactly what wave w % 4 of split w / 4 does in gemv_kernel (same tile columns
 // and order, same MFMA chains, same acc0 + acc1), so each split's sum over its four waves (in wave
@@ -780,6 +867,19 @@ bool fused_eligible(const GemvParams &p) {
          p.CG <= kFusedMaxColumns;
 }
 
+template <bool F16>
+hipError_t launch_batch(const GemvParams &p, hipStream_t stream) {
+  const int max_cols = (p.CG + p.ks - 1) / p.ks;
+  const size_t lds = (size_t)max_cols * ((p.tokens + 3) / 4) * 1024;
+  const dim3 grid((p.RG + kBatchWaves - 1) / kBatchWaves, p.ks);
+  if (p.lut) hipLaunchKernelGGL((gemv_batch_kernel<F16, true>), grid, dim3(64 * kBatchWaves), lds, stream, p);
+  else hipLaunchKernelGGL((gemv_batch_kernel<F16, false>), grid, dim3(64 * kBatchWaves), lds, stream, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  launch_splitk_reduce<F16, false>(p, stream);
+  return hipGetLastError();
+}
+
 template <bool F16, int LA, bool MULTI, bool F32OUT>
 hipError_t launch_variant(const GemvParams &p, hipStream_t stream) {
   if constexpr (!MULTI) {
@@ -851,6 +951,27 @@ bool gemv_fused_profitable(int RG, int CG, int ks, int cus) {
   if (ks < 2 || ks > kFusedMaxSplits || CG > kFusedMaxColumns) return false;
   const int tiles_per_wave = ((CG + ks - 1) / ks + kWaves - 1) / kWaves;
   return tiles_per_wave <= 8 && (RG <= cus || 2 * RG >= 3 * cus);
+}
+
+int gemv_batch_splits(int RG, int CG, int K, int64_t tokens, int cus) {
+  // From 4097 input features: below, the unsplit kernel's four waves a row group have few tiles each and
+  // the reduce launch costs more than it gains (us, unsplit against split: 2048 x 2048 at 8 tokens 5.5 / 5.9,
+  // 11008 x 2048 at 15 9.3 / 10.9; 1024 x 5120 at 8 9.0 / 7.5, 27648 x 5120 at 2 22.2 / 22.3 and at 15
+  // 46.0 / 28.5, 5120 x 27648 at 8 46.6 / 25.7).
+  if (tokens < 2 || tokens > 16 || CG <= 32 || tokens * K > 0x3FFFFFF0) return 0;
+  // About twelve waves a CU (16 to 32 were level to 25% slower: more partials); at most as many splits
+  // as keep the partials a quarter of the weights' bytes (ks * tokens * 4 against K / 2 / 4 per row);
+  // at least as many as the LDS needs.
+  const int waves = (RG + kBatchWaves - 1) / kBatchWaves * kBatchWaves;
+  int ks = (12 * cus + waves - 1) / waves;
+  ks = std::min(ks, std::max(1, (int)(K / (32 * tokens))));
+  const int max_cols = kBatchLdsBytes / (int)((tokens + 3) / 4 * 1024);
+  ks = std::min(std::max(ks, (CG + max_cols - 1) / max_cols), CG);
+  return ks <= 65535 && (int64_t)ks * CG <= 0x7FFFFFFF ? ks : 0;  // the grid, the kernel's 32-bit split arithmetic
+}
+
+hipError_t launch_gemv_batch(const GemvParams &p, hipStream_t stream) {
+  return p.f16 ? launch_batch<true>(p, stream) : launch_batch<false>(p, stream);
 }
 
 bool gemv_lookahead_supported(int la) { return la == 1 || la == 2 || la == 3 || la == 4 || la == 6 || la == 8; }

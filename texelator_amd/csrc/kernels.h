@@ -92,6 +92,10 @@ struct PrefillParams {
 // GEMV variants selected by the lookahead knob (number of 1 KiB tiles in flight per wave).
 bool gemv_lookahead_supported(int lookahead);
 hipError_t launch_gemv(const GemvParams &p, int lookahead, bool f32_out, hipStream_t stream);
+// K splits of the GEMV of 2 to 16 tokens (gemv_batch_kernel, then the split-K reduce), 0 where it does not
+// run; and the launch, with p.ks those splits and p.partials [ks][tokens][Mp].
+int gemv_batch_splits(int RG, int CG, int K, int64_t tokens, int cus);
+hipError_t launch_gemv_batch(const GemvParams &p, hipStream_t stream);
 hipError_t gemv_kernel_attributes(int lookahead, hipFuncAttributes *attr);
 // Workgroups of the single-token bf16 GEMV with this lookahead one CU holds at once, for a split of
 // `columns` tile columns (its x slice is dynamic LDS).
