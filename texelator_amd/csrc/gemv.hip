@@ -324,7 +324,9 @@ __device__ __forceinline__ TileRows tile_rows(const float4 *lut, uint4 tile) {
   const bool odd = threadIdx.x & 1;
   const float4 *half = lut + (threadIdx.x & 1);
   auto swap = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false); };
-  const uint32_t ra = palette_row(tile.x, tile.y), rb = palette_row(tile.z, tile.w);
+  // Past a wave's last tile the ring holds other bytes (TileStream::load), whose rows are fetched and never
+  // used: kept inside the 255 x 255 table.
+  const uint32_t ra = min(palette_row(tile.x, tile.y), 255u * 255u - 1u), rb = min(palette_row(tile.z, tile.w), 255u * 255u - 1u);
   const uint32_t pa = swap(ra), pb = swap(rb);
   return TileRows{half[2 * (size_t)(odd ? pa : ra)], half[2 * (size_t)(odd ? ra : pa)], half[2 * (size_t)(odd ? pb : rb)],
                   half[2 * (size_t)(odd ? rb : pb)]};
