@@ -134,7 +134,7 @@ int choose_splits(int RG, int CG, int cus) {
 
 // Workspace bytes of a prefill call (split-K partials), 0 if none.
 int64_t prefill_workspace_bytes(const Handle *h, int64_t tokens) {
-  const int ks = tx::prefill_splits(h->M, h->CG, tokens, h->cus);
+  const int ks = tx::prefill_splits(h->M, h->K, tokens, h->cus);
   return ks > 1 ? (int64_t)ks * tokens * h->Mp * (int64_t)sizeof(float) : 0;
 }
 
@@ -202,7 +202,7 @@ int run_prefill(Handle *h, int candidate, const void *x, bool f16, int64_t token
   p.RG = h->RG;
   p.CG = h->CG;
   p.tokens = (int)tokens;
-  p.ks = tx::prefill_splits(h->M, h->CG, tokens, h->cus);
+  p.ks = tx::prefill_splits(h->M, h->K, tokens, h->cus);
   if (tokens > (1 << 20)) return fail(TX_ERR_INVALID, "token count exceeds the prefill limit (1048576)");
   const int64_t need = prefill_workspace_bytes(h, tokens);
   if (need > 0) {
@@ -949,7 +949,7 @@ int tx_linear_swiglu_prefill(uint64_t value, const void *x, int64_t tokens, void
     return fail(TX_ERR_UNSUPPORTED, "linear_swiglu_prefill: the call is below the prefill threshold (use tx_linear_swiglu "
                                     "for one token, tx_linear + tx_swiglu otherwise)");
   const int candidate = prefill_choice(h, tokens);
-  if (!tx::prefill_swiglu_supported(candidate) || tx::prefill_splits(h->M, h->CG, tokens, h->cus) != 1)
+  if (!tx::prefill_swiglu_supported(candidate) || tx::prefill_splits(h->M, h->K, tokens, h->cus) != 1)
     return fail(TX_ERR_UNSUPPORTED, "linear_swiglu_prefill: this call's prefill runs the pair tile or the dense "
                                     "backend, or splits K (use tx_linear + tx_swiglu)");
   DeviceGuard guard(h->device);
@@ -975,7 +975,7 @@ int tx_linear_swiglu_prefill(uint64_t value, const void *x, int64_t tokens, void
 // (tx_prefill_split), as the prefill reduce sums and rounds them.
 tx::SplitSource prefill_split_source(const Handle *h, const void *partials, int64_t tokens) {
   return tx::SplitSource{static_cast<const float *>(partials), static_cast<const uint16_t *>(h->bias),
-                         tx::prefill_splits(h->M, h->CG, tokens, h->cus), h->Mp, (int)tokens, 1};
+                         tx::prefill_splits(h->M, h->K, tokens, h->cus), h->Mp, (int)tokens, 1};
 }
 
 int tx_prefill_split(uint64_t value, const void *x, int64_t tokens, void *workspace, int64_t workspace_bytes,
@@ -989,9 +989,12 @@ int tx_prefill_split(uint64_t value, const void *x, int64_t tokens, void *worksp
   if (tokens > (1 << 20)) return fail(TX_ERR_INVALID, "token count exceeds the prefill limit (1048576)");
   if (tokens < 2 || tokens < h->prefill_threshold)
     return fail(TX_ERR_UNSUPPORTED, "prefill_split: the call is below the prefill threshold (tx_linear runs the GEMV)");
-  const int candidate = prefill_choice(h, tokens);
+  // The split-group form sums its splits itself, so the default is the tile that leaves partials fastest.
+  const int candidate = h->prefill_backend == kDenseBackend || h->prefill_backend >= tx::kPrefillFirst
+                            ? prefill_choice(h, tokens)
+                            : tx::prefill_register_candidate(h->M, h->K, tokens, h->cus);
   if (candidate == kDenseBackend) return fail(TX_ERR_UNSUPPORTED, "prefill_split: the dense backend has no K splits");
-  const int ks = tx::prefill_splits(h->M, h->CG, tokens, h->cus);
+  const int ks = tx::prefill_splits(h->M, h->K, tokens, h->cus);
   if (ks == 1) return fail(TX_ERR_UNSUPPORTED, "prefill_split: this call does not split K (use tx_linear)");
   if (!workspace || workspace_bytes < prefill_workspace_bytes(h, tokens) || reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
     return fail(TX_ERR_INVALID, "prefill_split: workspace missing or too small (see tx_workspace_bytes)");

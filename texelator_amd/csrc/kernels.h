@@ -110,12 +110,15 @@ constexpr int kPrefillLast = 9;
 bool prefill_candidate_eligible(int candidate, int M, int K);
 // K splits of the prefill GEMM for a shape (the same for every candidate).
 // Default tile by shape (the autotuner's profile overrides it): measured best on the 27B-class
-// shapes -- small_32x128 up to 32 tokens, medium_64x128 up to 64, medium_128x128 below 256 (two
+// shapes -- small_32x128 up to 32 tokens, and up to 128 where its split-group form pays (prefill.hip),
+// else medium_64x128 up to 64, medium_128x128 below 256 (two
 // workgroups per CU, which hide each other's LDS and decode latency), from 256 tokens
 // large_256x128 (decode shared by wave pairs) when its workgroups make one round of the CUs at
-// least three quarters full.
+// least three quarters full. prefill_register_candidate: the same without the split-group form, for
+// callers that want the splits' partials (tx_prefill_split).
 int prefill_default_candidate(int M, int K, int64_t tokens, int cus);
-int prefill_splits(int M, int CG, int64_t tokens, int cus);
+int prefill_register_candidate(int M, int K, int64_t tokens, int cus);
+int prefill_splits(int M, int K, int64_t tokens, int cus);
 hipError_t launch_prefill(const PrefillParams &p, int candidate, hipStream_t stream);
 // Tile `candidate` (6-9) on a merged [gate | up] matrix (p.M = 2 * inter, inter a multiple of 16,
 // p.ks == 1, bf16) with a SwiGLU epilogue: p.y receives bf16 [tokens][inter], the bits of

@@ -635,15 +635,16 @@ __global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillParams p) {
   }
 }
 
-// Split-group tile (candidate 9 with exactly four K splits, up to 32 tokens, K a multiple of
-// 128): a workgroup holds the four splits of one (32-token tile, RBW x 32-row blocks), one per
+// Split-group tile (candidate 9 with exactly four K splits, up to 128 tokens, K a multiple of
+// 128): a workgroup holds the four splits of one (TBW x 32 tokens, RBW x 32 rows), one per
 // wave, and each wave runs its split on its own -- weights decoded in registers as in
 // prefill_kernel, activations staged by the wave itself into its own LDS buffers (direct
 // buffer-to-LDS loads, 1 KiB contiguous per load) half a step at a time -- so the K loop has no
 // workgroup barrier. With RBW = 2 a wave multiplies one staged activation slice by two row blocks
 // (two independent MFMA chains): the activations are read from L2 once per 64 rows instead of once
 // per 32, which was the kernel's bound (per K column, 32 tokens of bf16 activations are 64 bytes
-// against 16 bytes of weights in a 32-row block). At the end the four splits are summed in split order
+// against 16 bytes of weights in a 32-row block). With TBW of 2 or 3 a decoded weight is multiplied by that
+// many token blocks instead (wave_token_blocks). At the end the four splits are summed in split order
 // through LDS, as prefill_reduce_kernel sums them: no partials leave the workgroup and no reduce
 // kernel runs. Same lane layouts, K sets and order as prefill_kernel, hence the same bits.
 #ifndef TX_SMALL_WAVE
@@ -653,16 +654,17 @@ __global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillParams p) {
 #define TX_WAVE_RBW2_MIN_WGS 256
 #endif
 
-template <bool F16, bool LUT, int RBW>
+template <bool F16, bool LUT, int RBW, int TBW = 1>
 __global__ __launch_bounds__(kThreads) void prefill_wave_kernel(PrefillParams p) {
-  static_assert(RBW == 1 || RBW == 2, "one or two 32-row blocks per wave");
-  // Per wave, K columns 0-63 (xlo) and 64-127 (xhi) of a step for its 32 tokens: token row r takes
+  static_assert((RBW == 1 && TBW >= 1 && TBW <= 3) || (RBW == 2 && TBW == 1), "row and token blocks (of 32) per wave");
+  constexpr int BT = 32 * TBW;
+  // Per wave, K columns 0-63 (xlo) and 64-127 (xhi) of a step for its tokens: token row r takes
   // 128 bytes, its 16-byte slot q holds columns 8*(q ^ ((r >> 1) % 8)).. +7 of the half (the 16
   // rows one operand read serves per LDS pass then fall on distinct banks: even and odd rows sit in
   // opposite halves of the banks). The two halves are separate LDS objects, so the compiler can
   // tell reads of one from loads into the other.
-  __shared__ __attribute__((aligned(16))) uint16_t xlo[4][32 * 64];
-  __shared__ __attribute__((aligned(16))) uint16_t xhi[4][32 * 64];
+  __shared__ __attribute__((aligned(16))) uint16_t xlo[4][BT * 64];
+  __shared__ __attribute__((aligned(16))) uint16_t xhi[4][BT * 64];
   __shared__ __attribute__((aligned(16))) PaletteTableStorage tables;
 
   const int lane = threadIdx.x & 63;
@@ -671,13 +673,13 @@ __global__ __launch_bounds__(kThreads) void prefill_wave_kernel(PrefillParams p)
   const int h = lane >> 5;
   const int row_blocks = (p.M + 31) / 32;
   const int row_groups = (row_blocks + RBW - 1) / RBW;
-  const int wgs = row_groups * ((p.tokens + 31) / 32);
+  const int wgs = row_groups * ((p.tokens + BT - 1) / BT);
   const int per_xcd = (wgs + kXcds - 1) / kXcds;
   const int q = (int)(blockIdx.x % kXcds) * per_xcd + (int)(blockIdx.x / kXcds);
   if (q >= wgs) return;
   if constexpr (!LUT) copy_seed_tables(tables, split, lane, kThreads / 64);
   const int rg = q % row_groups;
-  const int t0 = (q / row_groups) * 32;
+  const int t0 = (q / row_groups) * BT;
   const int c_begin = (int)((uint32_t)split * (uint32_t)p.CG / 4u);
   const int nc = (int)((uint32_t)(split + 1) * (uint32_t)p.CG / 4u) - c_begin;
 
@@ -729,9 +731,9 @@ __global__ __launch_bounds__(kThreads) void prefill_wave_kernel(PrefillParams p)
   // (l % 8) ^ (((8v + l / 8) >> 1) % 8). Rows past the tokens repeat the last token (never stored).
   const uint16_t *x = static_cast<const uint16_t *>(p.x);
   const int srow = lane >> 3;  // row within the load's eight
-  uint32_t row_off[4];         // byte offsets of this lane's four token rows and chunks
+  uint32_t row_off[4 * TBW];   // byte offsets of this lane's token rows and chunks
 #pragma unroll
-  for (int v = 0; v < 4; ++v)
+  for (int v = 0; v < 4 * TBW; ++v)
     row_off[v] = 2u * ((uint32_t)min(t0 + 8 * v + srow, p.tokens - 1) * (uint32_t)p.K +
                        8u * (uint32_t)((lane & 7) ^ ((4 * v + (srow >> 1)) & 7)));
   const int64_t x_bytes = ((int64_t)p.tokens * p.K - (int64_t)c_begin * kTileK) * 2;
@@ -741,13 +743,15 @@ __global__ __launch_bounds__(kThreads) void prefill_wave_kernel(PrefillParams p)
   auto stage = [&](uint16_t *buf, int j, int hf) {
     const int off = __builtin_amdgcn_readfirstlane((j * kTileK + 64 * hf) * 2);
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xrsrc, (__attribute__((address_space(3))) void *)(buf + 8 * v * 64), 16,
-                                               row_off[v], off, 0, 0);
+    for (int v = 0; v < 4 * TBW; ++v) {
+      uint32_t row = row_off[v];  // an element of a dependent array as the operand drops the host stub silently
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xrsrc, (__attribute__((address_space(3))) void *)(buf + 8 * v * 64), 16, row,
+                                               off, 0, 0);
+    }
   };
   // B operand of MFMA 4*hf + s (s < 4): columns 32h + 16*(s>>1) + 8*(s&1) .. +7 of half hf.
-  auto read_b = [&](const uint16_t *buf, int s) {
-    return *reinterpret_cast<const u32x4 *>(buf + r32 * 64 + 8 * ((4 * h + s) ^ ((r32 >> 1) & 7)));
+  auto read_b = [&](const uint16_t *buf, int tb, int s) {
+    return *reinterpret_cast<const u32x4 *>(buf + (32 * tb + r32) * 64 + 8 * ((4 * h + s) ^ ((r32 >> 1) & 7)));
   };
 
   uint16_t *mylo = xlo[split];
@@ -761,11 +765,13 @@ __global__ __launch_bounds__(kThreads) void prefill_wave_kernel(PrefillParams p)
     __syncthreads();  // the seed tables
   }
 
-  f32x16 acc[RBW];
+  f32x16 acc[RBW][TBW];
 #pragma unroll
   for (int b = 0; b < RBW; ++b)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
+    for (int tb = 0; tb < TBW; ++tb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[b][tb][r] = 0.f;
 
   // Block jj of row block b's weight tile into that block's MFMAs 2jj, 2jj + 1.
   auto words = [](const Tiles &tile, int b, int jj, uint32_t &wa, uint32_t &wb) {
@@ -775,7 +781,7 @@ __global__ __launch_bounds__(kThreads) void prefill_wave_kernel(PrefillParams p)
   };
   // Block jj of row block b's weight tile into that block's MFMAs 2jj, 2jj + 1 (palette seeds
   // already read from the LDS tables, or the palette row from p.lut).
-  auto block = [&](const Tiles &tile, int b, int jj, const Seeds &sd, const u32x4 &b0, const u32x4 &b1) {
+  auto block = [&](const Tiles &tile, int b, int jj, const Seeds &sd, const u32x4 (&bv)[TBW][4]) {
     uint32_t wa, wb, d[8];
     words(tile, b, jj, wa, wb);
     if constexpr (LUT) {
@@ -784,23 +790,29 @@ __global__ __launch_bounds__(kThreads) void prefill_wave_kernel(PrefillParams p)
     } else {
       decode_from_seeds_mode<F16>(sd.base, sd.end, sd.step, sd.mode, wa, wb, scale[b], pm[b], d);
     }
-    acc[b] = mfma<F16>(u32x4{d[0], d[1], d[2], d[3]}, b0, acc[b]);
-    acc[b] = mfma<F16>(u32x4{d[4], d[5], d[6], d[7]}, b1, acc[b]);
+    const int s = 2 * (jj & 1);  // the half's operands
+#pragma unroll
+    for (int tb = 0; tb < TBW; ++tb) acc[b][tb] = mfma<F16>(u32x4{d[0], d[1], d[2], d[3]}, bv[tb][s], acc[b][tb]);
+#pragma unroll
+    for (int tb = 0; tb < TBW; ++tb) acc[b][tb] = mfma<F16>(u32x4{d[4], d[5], d[6], d[7]}, bv[tb][s + 1], acc[b][tb]);
   };
   // Step j multiplies weight tiles `cur` (loaded during step j - 1) and loads tiles j + 1 into
   // `next`. Each half buffer is read into registers together with the palette seeds of the half's
   // blocks (one LDS wait for both, so no seed read waits inside a decode), then refilled with the
   // next step's half while this step's blocks are decoded and multiplied. Loads are issued low
-  // half (4), weights (2 RBW), high half (4): 4 + 2 RBW later loads stay in flight at each half
+  // half (4 TBW), weights (2 RBW), high half (4 TBW): 4 TBW + 2 RBW later loads stay in flight at each half
   // buffer's wait.
-  constexpr int kLaterLoads = 4 + 2 * RBW;
+  constexpr int kLaterLoads = 4 * TBW + 2 * RBW;
+  static_assert(kLaterLoads < 16, "the low four bits of the wait's vmcnt");
   constexpr int kHalfWait = 0x0F70 | kLaterLoads;  // vmcnt(kLaterLoads), lgkmcnt and expcnt free
   auto half = [&](int jn, int jt, int hf, uint16_t *buf, const Tiles &cur, Tiles &next) {
-    u32x4 bv[4];
+    u32x4 bv[TBW][4];
     Seeds sd[2][RBW];
     __builtin_amdgcn_s_waitcnt(kHalfWait);  // this half of step j has landed
 #pragma unroll
-    for (int s = 0; s < 4; ++s) bv[s] = read_b(buf, s);
+    for (int tb = 0; tb < TBW; ++tb)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) bv[tb][s] = read_b(buf, tb, s);
     if constexpr (!LUT) {
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj)
@@ -819,7 +831,7 @@ __global__ __launch_bounds__(kThreads) void prefill_wave_kernel(PrefillParams p)
 #pragma unroll
     for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
-      for (int b = 0; b < RBW; ++b) block(cur, b, 2 * hf + jj, sd[jj][b], bv[2 * jj], bv[2 * jj + 1]);
+      for (int b = 0; b < RBW; ++b) block(cur, b, 2 * hf + jj, sd[jj][b], bv);
   };
   auto step = [&](int j, const Tiles &cur, Tiles &next) {
     const int jn = min(j + 1, nc - 1);
@@ -833,44 +845,44 @@ __global__ __launch_bounds__(kThreads) void prefill_wave_kernel(PrefillParams p)
   }
   if (j < nc) step(j, ta, tb);
 
-  // acc[b][r] = D[row 8(r/4) + 4h + r%4 of block b][token t0 + r32]. The four splits are summed in
-  // split order from zero through each wave's buffers (after its last refill has landed), two
-  // blocks at a time (block 2i in the low buffer, 2i + 1 in the high one); wave w finishes rows
+  // acc[b][tb][r] = D[row 8(r/4) + 4h + r%4 of block b][token t0 + 32 tb + r32]. The four splits are summed
+  // in split order from zero through each wave's buffers (after its last refill has landed): row block
+  // 0 in the low buffer, row block 1 in the high one, token block tb at 4 KiB tb; wave w finishes rows
   // 8w + 4h .. + 3 of each block.
-  const int t = t0 + r32;
   const uint16_t *bias = static_cast<const uint16_t *>(p.bias);
-  uint16_t *y = static_cast<uint16_t *>(p.y) + (size_t)min(t, p.tokens - 1) * p.M;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-  for (int b0 = 0; b0 < RBW; b0 += 2) {
-    if (b0 > 0) __syncthreads();  // the previous pair's sums are read
+  for (int b = 0; b < RBW; ++b)
 #pragma unroll
-    for (int b = b0; b < b0 + 2 && b < RBW; ++b) {
-      float *mine = reinterpret_cast<float *>(b == b0 ? mylo : myhi);
+    for (int tb = 0; tb < TBW; ++tb) {
+      float *mine = reinterpret_cast<float *>(b == 0 ? mylo : myhi) + tb * 1024;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mine[r * 64 + lane] = acc[b][r];
+      for (int r = 0; r < 16; ++r) mine[r * 64 + lane] = acc[b][tb][r];
     }
-    __syncthreads();
-    if (t < p.tokens) {
+  __syncthreads();
 #pragma unroll
-      for (int b = b0; b < b0 + 2 && b < RBW; ++b) {
-        const int n = n0[b] + 8 * split + 4 * h;
-        uint32_t out[4];
+  for (int tb = 0; tb < TBW; ++tb) {
+    const int t = t0 + 32 * tb + r32;
+    if (t >= p.tokens) continue;
+    uint16_t *y = static_cast<uint16_t *>(p.y) + (size_t)t * p.M;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float total = 0.f;
+    for (int b = 0; b < RBW; ++b) {
+      const int n = n0[b] + 8 * split + 4 * h;
+      uint32_t out[4];
 #pragma unroll
-          for (int s = 0; s < 4; ++s)
-            total += reinterpret_cast<const float *>(b == b0 ? xlo[s] : xhi[s])[(4 * split + r) * 64 + lane];
-          out[r] = n + r < p.M ? out_bits<F16>(total, bias, n + r) : 0u;
-        }
-        if (n + 3 < p.M && ((reinterpret_cast<uintptr_t>(y + n) & 7) == 0)) {
-          *reinterpret_cast<uint2 *>(y + n) = make_uint2(out[0] | (out[1] << 16), out[2] | (out[3] << 16));
-        } else {
+      for (int r = 0; r < 4; ++r) {
+        float total = 0.f;
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (n + r < p.M) y[n + r] = (uint16_t)out[r];
-        }
+        for (int s = 0; s < 4; ++s)
+          total += reinterpret_cast<const float *>(b == 0 ? xlo[s] : xhi[s])[tb * 1024 + (4 * split + r) * 64 + lane];
+        out[r] = n + r < p.M ? out_bits<F16>(total, bias, n + r) : 0u;
+      }
+      if (n + 3 < p.M && ((reinterpret_cast<uintptr_t>(y + n) & 7) == 0)) {
+        *reinterpret_cast<uint2 *>(y + n) = make_uint2(out[0] | (out[1] << 16), out[2] | (out[3] << 16));
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (n + r < p.M) y[n + r] = (uint16_t)out[r];
       }
     }
   }
@@ -1568,31 +1580,64 @@ __global__ __launch_bounds__(kWideThreads) void prefill_wide_kernel(PrefillParam
 }
 
 // y[t][m] = round(sum over splits in order of partials[s][t][m]), then the bias with a second
-// rounding (the reference's epilogue order); bf16, or fp16 with F16.
-// KS > 0: exactly KS splits, every partial loaded before the first add (a runtime loop waited
-// for memory once per split); KS = 0: any count.
+// rounding (the reference's epilogue order); bf16, or fp16 with F16. A thread takes four columns.
+// KS > 0: exactly KS splits, every partial loaded before the first add; KS = 0: any count, eight loads
+// at a time (a loop over single loads waited for memory once per split: 5 to 25 splits are usual).
+constexpr int kReduceMaxKS = 16;
 template <bool F16, int KS>
 __global__ __launch_bounds__(256) void prefill_reduce_kernel(PrefillParams p) {
-  const int m = blockIdx.x * 256 + threadIdx.x;
+  const int m = (blockIdx.x * 256 + threadIdx.x) * 4;
   const int t = blockIdx.y;
   if (m >= p.M) return;
-  // the bias goes out with the partials (from a valid address whether or not there is one)
-  const uint16_t b = (p.bias ? static_cast<const uint16_t *>(p.bias) : reinterpret_cast<const uint16_t *>(p.partials))[m];
-  float total = 0.f;
-  const float *src = p.partials + (size_t)t * p.Mp + m;
-  const size_t stride = (size_t)p.tokens * p.Mp;
+  const float4 *src = reinterpret_cast<const float4 *>(p.partials + (size_t)t * p.Mp + m);  // Mp is a multiple of 16
+  const size_t stride = (size_t)p.tokens * p.Mp / 4;
+  float4 total = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto add = [&](const float4 &v) {
+    total.x += v.x;
+    total.y += v.y;
+    total.z += v.z;
+    total.w += v.w;
+  };
+  uint16_t b[4] = {0, 0, 0, 0};
+  if (p.bias) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b[e] = static_cast<const uint16_t *>(p.bias)[min(m + e, p.M - 1)];
+  }
   if constexpr (KS > 0) {
-    float v[KS];
+    float4 v[KS];
 #pragma unroll
     for (int s = 0; s < KS; ++s) v[s] = src[s * stride];
+    __builtin_amdgcn_sched_barrier(0);  // every load issued before the first add
 #pragma unroll
-    for (int s = 0; s < KS; ++s) total += v[s];
+    for (int s = 0; s < KS; ++s) add(v[s]);
   } else {
-    for (int s = 0; s < p.ks; ++s) total += src[s * stride];
+    constexpr int kGroup = 8;
+    for (int s0 = 0; s0 < p.ks; s0 += kGroup) {
+      float4 v[kGroup];
+#pragma unroll
+      for (int u = 0; u < kGroup; ++u) v[u] = src[(size_t)min(s0 + u, p.ks - 1) * stride];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < kGroup; ++u)
+        if (s0 + u < p.ks) add(v[u]);
+    }
   }
-  float out = round_out<F16>(total);
-  if (p.bias) out += half_bits_to_float<F16>(b);
-  store_out<F16>(p.y, (size_t)t * p.M + m, out);
+  const float sums[4] = {total.x, total.y, total.z, total.w};
+  uint16_t out[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float v = round_out<F16>(sums[e]);
+    if (p.bias) v += half_bits_to_float<F16>(b[e]);
+    out[e] = F16 ? __builtin_bit_cast(uint16_t, (_Float16)v) : to_bf(v);
+  }
+  uint16_t *y = static_cast<uint16_t *>(p.y) + (size_t)t * p.M + m;
+  if (m + 3 < p.M && (reinterpret_cast<uintptr_t>(y) & 7) == 0) {
+    *reinterpret_cast<uint2 *>(y) = make_uint2((uint32_t)out[0] | ((uint32_t)out[1] << 16), (uint32_t)out[2] | ((uint32_t)out[3] << 16));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (m + e < p.M) y[e] = out[e];
+  }
 }
 
 struct Candidate {
@@ -1605,14 +1650,14 @@ struct Candidate {
 };
 
 // The ordered reduction of the split-K partials, after the tile kernel.
-template <bool F16>
+template <bool F16, int KS = 2>
 void launch_reduce_as(const PrefillParams &p, hipStream_t stream) {
-  const dim3 grid((p.M + 255) / 256, p.tokens);
-  switch (p.ks) {
-    case 2: hipLaunchKernelGGL((prefill_reduce_kernel<F16, 2>), grid, dim3(256), 0, stream, p); break;
-    case 3: hipLaunchKernelGGL((prefill_reduce_kernel<F16, 3>), grid, dim3(256), 0, stream, p); break;
-    case 4: hipLaunchKernelGGL((prefill_reduce_kernel<F16, 4>), grid, dim3(256), 0, stream, p); break;
-    default: hipLaunchKernelGGL((prefill_reduce_kernel<F16, 0>), grid, dim3(256), 0, stream, p); break;
+  const dim3 grid((p.M + 1023) / 1024, p.tokens);
+  if constexpr (KS <= kReduceMaxKS) {
+    if (p.ks == KS) hipLaunchKernelGGL((prefill_reduce_kernel<F16, KS>), grid, dim3(256), 0, stream, p);
+    else launch_reduce_as<F16, KS + 1>(p, stream);
+  } else {
+    hipLaunchKernelGGL((prefill_reduce_kernel<F16, 0>), grid, dim3(256), 0, stream, p);
   }
 }
 
@@ -1693,6 +1738,39 @@ hipError_t launch_tile(const PrefillParams &p, hipStream_t stream) {
   return launch_reduce(p, stream);
 }
 
+// 32-token blocks per wave of the split-group tile: the fewest whose workgroups make one round of the CUs
+// (more blocks decode each weight for more tokens, but a half-empty chip waits longer on each wave:
+// 2048 x 2048 at 128 tokens 7.2 us with one block, 8.2 with two, 10.0 with three; 5120 x 5120 at 96 tokens
+// 19.4, 26.2 and 19.2), and two where none makes it (8192 x 3072 at 128 tokens 20.2, 18.9 and 26.1).
+int wave_token_blocks(int row_blocks, int token_tiles, int cus) {
+  for (int tbw = 1; tbw <= 3; ++tbw)
+    if ((int64_t)row_blocks * ((token_tiles + tbw - 1) / tbw) <= cus) return tbw;
+  return token_tiles == 1 ? 1 : 2;
+}
+
+constexpr int kWaveCus = 256;           // MI355X
+constexpr int kWaveMaxTokens = 128;     // four token tiles
+constexpr int kWaveMinColumns = 16, kWaveMaxColumns = 64;  // K tiles of 128
+
+// Whether the split-group tile with four K splits is the default for a shape whose K is split at all. Four waves
+// of a workgroup share one row block, so it wants K short enough that a quarter of it is no long chain
+// (5120 x 27648 at 32 tokens 40.5 us against 35.9 of the 32-token tile with 12 splits), enough row blocks
+// (1024 x 5120 at 16 tokens 9.5 us with the finer splits of prefill_splits), and workgroups that fill one
+// round of the CUs, or two of them by two thirds. Before and now: 2048 x 2048 at 128 tokens 13.9 -> 7.2 us,
+// 7168 x 5120 at 64 23.8 -> 15.6 and at 128 32.6 -> 27.3, 8192 x 3072 at 96 23.8 -> 14.3, 11008 x 2048 at 64
+// 17.6 -> 12.9, 5120 x 5120 at 20 14.3 -> 10.9 and at 77 21.8 -> 17.9. Outside: 5120 x 5120 at 128 tokens (320
+// workgroups) 26.8 against 25.0, 27648 x 5120 at 64 (864) 50.4 against 43.9.
+bool wave_tile_pays(int M, int K, int64_t tokens, int cus) {
+  const int CG = (K + kTileK - 1) / kTileK;
+  if (tokens > kWaveMaxTokens || K % kTileK != 0 || CG < kWaveMinColumns || CG > kWaveMaxColumns) return false;
+  const int64_t row_blocks = (M + 31) / 32, token_tiles = (tokens + 31) / 32;
+  if (row_blocks * token_tiles < 64) return false;
+  if (token_tiles == 1) return true;
+  const int tbw = wave_token_blocks((int)row_blocks, (int)token_tiles, cus);
+  const int64_t wgs = row_blocks * ((token_tiles + tbw - 1) / tbw);
+  return wgs <= cus || (wgs <= 2 * (int64_t)cus && 3 * wgs >= 4 * (int64_t)cus);
+}
+
 template <bool F16, bool LUT>
 void launch_wave_as(const PrefillParams &p, hipStream_t stream) {
   // Two row blocks per wave when that still gives every CU of the MI355X (256) a workgroup
@@ -1700,22 +1778,22 @@ void launch_wave_as(const PrefillParams &p, hipStream_t stream) {
   // workgroups, 35.9 us; four, 216 workgroups, 31.5 us).
   const int row_blocks = (p.M + 31) / 32, token_tiles = (p.tokens + 31) / 32;
   const int wide = (row_blocks + 1) / 2 * token_tiles;
-  if (wide >= TX_WAVE_RBW2_MIN_WGS) {
-    hipLaunchKernelGGL((prefill_wave_kernel<F16, LUT, 2>), dim3((wide + kXcds - 1) / kXcds * kXcds), dim3(kThreads), 0,
-                       stream, p);
-  } else {
-    const int wgs = row_blocks * token_tiles;
-    hipLaunchKernelGGL((prefill_wave_kernel<F16, LUT, 1>), dim3((wgs + kXcds - 1) / kXcds * kXcds), dim3(kThreads), 0,
-                       stream, p);
-  }
+  const int tbw = wave_token_blocks(row_blocks, token_tiles, kWaveCus);
+  const bool two_rows = token_tiles == 1 && wide >= TX_WAVE_RBW2_MIN_WGS;
+  const int wgs = two_rows ? wide : row_blocks * ((token_tiles + tbw - 1) / tbw);
+  const dim3 grid((wgs + kXcds - 1) / kXcds * kXcds), threads(kThreads);
+  if (two_rows) hipLaunchKernelGGL((prefill_wave_kernel<F16, LUT, 2, 1>), grid, threads, 0, stream, p);
+  else if (tbw == 1) hipLaunchKernelGGL((prefill_wave_kernel<F16, LUT, 1, 1>), grid, threads, 0, stream, p);
+  else if (tbw == 2) hipLaunchKernelGGL((prefill_wave_kernel<F16, LUT, 1, 2>), grid, threads, 0, stream, p);
+  else hipLaunchKernelGGL((prefill_wave_kernel<F16, LUT, 1, 3>), grid, threads, 0, stream, p);
 }
 
 // Candidate 9: the split-group tile where a workgroup holds all four K splits of a 32- or 64-row
-// block (exactly four splits, up to 32 tokens, K a multiple of 128, partials not wanted by the
+// block (exactly four splits, up to 128 tokens, K a multiple of 128, partials not wanted by the
 // caller): no reduce launch. Elsewhere the register-decoding 32-token tile, which was faster with
 // split partials (down 27648 -> 5120 at 32 tokens: 40.1 vs 42.0 us). Both give the same bits.
 hipError_t launch_small(const PrefillParams &p, hipStream_t stream) {
-  if (!TX_SMALL_WAVE || p.ks != 4 || p.tokens > 32 || p.K % kTileK != 0 || p.no_reduce)
+  if (!TX_SMALL_WAVE || p.ks != 4 || p.tokens > kWaveMaxTokens || p.K % kTileK != 0 || p.no_reduce)
     return launch_tile<1, 1, TX_PREFILL_LA_PLAIN, false>(p, stream);
   if (p.lut) {
     if (p.f16) launch_wave_as<true, true>(p, stream);
@@ -1775,7 +1853,8 @@ const std::array<int, kPrefillLast - kPrefillFirst + 1> &resident_per_cu() {
 
 }  // namespace
 
-int prefill_default_candidate(int M, int K, int64_t tokens, int cus) {
+// The default tile where the split-group tile is not taken, and the splits it asks for.
+int prefill_register_candidate(int M, int K, int64_t tokens, int cus) {
   if (tokens <= 32) return 9;   // small_32x128x128
   if (tokens <= 64) return 8;   // medium_64x128x128
   if (tokens < 256) return 6;   // medium_128x128x128
@@ -1806,20 +1885,32 @@ int prefill_default_candidate(int M, int K, int64_t tokens, int cus) {
   return 4 * items * splits(items) >= 3 * (int64_t)cus ? 5 : 6;
 }
 
-int prefill_splits(int M, int CG, int64_t tokens, int cus) {
+int prefill_splits(int M, int K, int64_t tokens, int cus) {
   // Candidate-independent, so that every tile gives the same sums, and sized for the default tile
   // of this shape: as many splits as keep all of its workgroups resident at once, each split at
   // least 8 tile columns long, partials at most 32 MiB.
-  const int dc = prefill_default_candidate(M, CG * kTileK, tokens, cus);
+  const int CG = (K + kTileK - 1) / kTileK;
+  const int dc = prefill_register_candidate(M, K, tokens, cus);
   const Candidate *c = find(dc);
   const int64_t items = ((M + c->bn - 1) / c->bn) * ((tokens + c->bt - 1) / c->bt);
   const int64_t slots = (int64_t)resident_per_cu()[dc - kPrefillFirst] * cus;
   int64_t ks = std::max<int64_t>(1, slots / items);
-  ks = std::min<int64_t>(ks, std::max(1, CG / 8));
+  const int64_t coarse = std::max(1, CG / 8);
+  // Below 256 tokens a grid that leaves CUs idle is split down to 4 columns, to one workgroup a CU (more, and
+  // from 256 tokens any, cost as much in partials: level or slower). 2048 x 2048 at 16 tokens 12.5 -> 6.7 us,
+  // 1024 x 5120 at 16 12.6 -> 9.5, 3000 x 4848 at 77 20.2 -> 17.9. A K that was not split stays whole.
+  const int64_t fine = tokens < 256 && coarse > 1 ? std::min<int64_t>(CG / 4, cus / items) : 1;
+  ks = std::min(ks, std::max(coarse, fine));
+  if (ks > 1 && wave_tile_pays(M, K, tokens, cus)) ks = 4;
   const int64_t cap = std::max<int64_t>(1, (int64_t(32) << 20) / (tokens * (int64_t)((M + 15) / 16 * 16) * 4));
   ks = std::min(ks, cap);
   ks = std::min<int64_t>(ks, std::max(1, 0x7FFFFFFF / std::max(CG, 1)));  // the kernels' 32-bit split arithmetic
   return (int)std::max<int64_t>(1, ks);
+}
+
+int prefill_default_candidate(int M, int K, int64_t tokens, int cus) {
+  if (tokens <= kWaveMaxTokens && wave_tile_pays(M, K, tokens, cus) && prefill_splits(M, K, tokens, cus) == 4) return 9;
+  return prefill_register_candidate(M, K, tokens, cus);
 }
 
 bool prefill_candidate_eligible(int candidate, int M, int K) {
