@@ -584,6 +584,7 @@ __global__ __launch_bounds__(64 * kBatchWaves, LUT ? 4 : 6) void gemv_batch_kern
   uint4 ring[R];
 #pragma unroll
   for (int u = 0; u < LA; ++u) ring[u] = stream.load(u, nc, 1);
+  if constexpr (LUT) ring[LA] = make_uint4(0u, 0u, 0u, 0u);  // with fewer than R tiles its rows are fetched all the same
   const int i = lane & 15, kg = lane >> 4;
   const float scale = p.scales[gc * kTileRows + i];
 
