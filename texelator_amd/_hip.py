@@ -38,10 +38,14 @@ def _require(condition: bool, message: str) -> None:
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
+def _stream_address(device: torch.device) -> int:
     if _raw_stream is not None:
-        return ctypes.c_void_p(_raw_stream(device.index if device.index is not None else torch.cuda.current_device()))
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+        return _raw_stream(device.index if device.index is not None else torch.cuda.current_device())
+    return torch.cuda.current_stream(device).cuda_stream
+
+
+def _stream(device: torch.device) -> ctypes.c_void_p:
+    return ctypes.c_void_p(_stream_address(device))
 
 
 def _aligned(x: torch.Tensor) -> torch.Tensor:
@@ -55,16 +59,11 @@ def workspace_bytes(handle: int, tokens: int) -> int:
     return int(out.value)
 
 
-def _workspace(handle: int, tokens: int, device: torch.device, linear: bool = False):
+def _workspace(handle: int, tokens: int, device: torch.device):
     """Stream-ordered scratch from the caching allocator (None when the shape needs none): the
-    prefill split-K partials, or (``linear``) those of a GEMV of one or a few tokens, so that calls on
-    one handle from several streams never share the handle's own buffer."""
-    nbytes = 0
-    if tokens >= 1:
-        out = ctypes.c_int64(0)
-        query = _lib.load().tx_linear_workspace_bytes if linear else _lib.load().tx_workspace_bytes
-        check(query(handle, tokens, ctypes.byref(out)))
-        nbytes = out.value
+    prefill split-K partials, or a one-token GEMV's, so that calls on one handle from several
+    streams never share the handle's own buffer."""
+    nbytes = workspace_bytes(handle, tokens) if tokens >= 1 else 0
     if nbytes == 0:
         return None, ctypes.c_void_p(None), 0
     ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
@@ -174,16 +173,23 @@ def linear(handle: int, x: torch.Tensor) -> torch.Tensor:
              "input must be contiguous CUDA FP16 or BF16")
     m, k = shape(handle)
     _require(x.dim() >= 1 and x.size(-1) == k, "input shape/device mismatch")
-    out_shape = list(x.shape)
+    device, out_shape = x.device, list(x.shape)
     out_shape[-1] = m
-    y = torch.empty(out_shape, dtype=x.dtype, device=x.device)
+    y = torch.empty(out_shape, dtype=x.dtype, device=device)
     x = _aligned(x)
-    tokens = x.numel() // k
-    ws, ws_ptr, ws_bytes = _workspace(handle, tokens, x.device, linear=True)
-    check(_lib.load().tx_linear(handle, ctypes.c_void_p(x.data_ptr()), _DTYPE_CODE[x.dtype], x.numel(),
-                                x.size(-1), x.device.index, ctypes.c_void_p(y.data_ptr()), ws_ptr, ws_bytes,
-                                _stream(x.device)))
-    del ws
+    numel = x.numel()
+    # Scratch as in _workspace, of the size tx_linear itself can use.
+    lib, ws, ws_bytes = _lib.load(), None, 0
+    if numel:
+        out = ctypes.c_int64(0)
+        check(lib.tx_linear_workspace_bytes(handle, numel // k, out))
+        ws_bytes = out.value
+        if ws_bytes:
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+    # Plain integers for pointers and no pointer object for the size: a 256 x 2048 linear, host bound,
+    # 9.4 us a call with an object per argument, 9.0 without.
+    check(lib.tx_linear(handle, x.data_ptr(), _DTYPE_CODE[x.dtype], numel, k, device.index, y.data_ptr(),
+                        None if ws is None else ws.data_ptr(), ws_bytes, _stream_address(device)))
     return y
 
 
