@@ -71,3 +71,30 @@ def test_k_that_was_whole_stays_whole(ext):
         assert [splits(ext, handle, 2048, t) for t in (2, 32, 33, 128, 200)] == [0] * 5
     finally:
         ext.free(handle)
+
+
+@pytest.mark.parametrize("tokens", [256, 257, 384, 385, 513, 640, 767, 768])
+@pytest.mark.parametrize("m,mode", [(3072, "bf16"), (3000, "f16_bias")])
+def test_sides_of_the_large_tiles_padding_rule(ext, oracle_threads, m, mode, tokens):
+    """Where the 256- and 512-token tiles would be mostly padding at their end the 128-token tile takes the call, with
+    its own K splits: the default is every tile's bits, and rows at both ends match float64 (bound as above)."""
+    handle, blocks, scales, bias, _ = pack(ext, m, 4096, mode)
+    x = (f16_vector if mode.startswith("f16") else bf16_vector)((tokens, 4096), tokens)
+    try:
+        got = ext.linear(handle, x.cuda())
+        for candidate in range(5, 10):
+            assert torch.equal(ext.prefill(handle, candidate, x.cuda()), got), candidate
+    finally:
+        ext.free(handle)
+    rows = np.r_[0:33, m - 33:m]
+    blocks, scales = blocks.reshape(m, -1)[rows], scales[rows]
+    if mode == "f16_bias":
+        want = x.double().numpy() @ bc4.decode_f16_bits(blocks, scales).view(np.float16).astype(np.float64).T
+    else:
+        want = clib.gemm_f64(bf16_bits(x), clib.decode_bf16_bits(blocks, scales))
+    half_ulp = 2 ** -11 if mode == "f16_bias" else 2 ** -8
+    bound = 1e-3 * np.maximum(np.abs(want), np.sqrt(np.mean(want ** 2))) + half_ulp * np.abs(want)
+    if bias is not None:
+        want = want + bias.double().numpy()[None, rows]
+        bound = bound + half_ulp * np.abs(want) * 1.01
+    assert (np.abs(want - got[:, rows].double().cpu().numpy()) <= bound).all()

@@ -1866,10 +1866,9 @@ int prefill_register_candidate(int M, int K, int64_t tokens, int cus) {
     ks = std::min<int64_t>(ks, std::max(1, CG / 8));
     return std::min(ks, std::max<int64_t>(1, (int64_t(32) << 20) / (tokens * (int64_t)((M + 15) / 16 * 16) * 4)));
   };
-  // The 512-token wide tile from 384 tokens (at most a quarter of its MFMA work past the
-  // tokens) when its workgroups make one round of the CUs at least three quarters full, or
+  // The 512-token wide tile where at most a quarter of its MFMA work is past the tokens, when its workgroups make one round of the CUs at least three quarters full, or
   // several rounds at least four fifths full on average.
-  if (tokens >= 384) {
+  if (4 * tokens >= 3 * 512 * ((tokens + 511) / 512)) {
     const int64_t wi = (int64_t)((M + 127) / 128) * ((tokens + 511) / 512);
     if (wi > (int64_t)cus) {
       if (5 * wi >= 4 * (int64_t)cus * ((wi + cus - 1) / cus)) return 7;
@@ -1882,6 +1881,14 @@ int prefill_register_candidate(int M, int K, int64_t tokens, int cus) {
   // finer grain fills sparse grids and the last of several rounds better.
   const int64_t items = (int64_t)((M + 127) / 128) * ((tokens + 255) / 256);
   if (items > (int64_t)cus) return 6;
+  // Where the last 256 tokens are at most half full, the 128x128 tile (two workgroups a CU) has less padding, if
+  // its workgroups make at least one and a quarter rounds of the CUs. Before and now, with the wide tile's
+  // three-quarters rule above: 5120 x 5120 at 320 tokens 46.7 -> 42.3 us, 5120 x 27648 154.7 -> 132.1, 13824 x 5120
+  // 85.5 -> 81.5; at 520 tokens 4096 x 4096 58.3 -> 40.5, 27648 x 5120 269.1 -> 211.4. Below the line 3000 x 4848
+  // at 333 tokens in fp16 (288 workgroups) 33.2 us, 33.7 on the 128x128 tile.
+  const int64_t fine = (int64_t)((M + 127) / 128) * ((tokens + 127) / 128);
+  const int64_t fine_ks = std::min<int64_t>(std::max<int64_t>(1, 2 * (int64_t)cus / fine), std::max(1, CG / 8));
+  if ((tokens - 1) % 256 < 128 && 4 * fine * fine_ks >= 5 * (int64_t)cus) return 6;
   return 4 * items * splits(items) >= 3 * (int64_t)cus ? 5 : 6;
 }
 
