@@ -66,6 +66,20 @@ def test_encoder_kernel_on_edge_rows(ext, palette):
     assert torch.equal(blocks, want_blocks)
 
 
+@pytest.mark.parametrize("signs", ["some", "all"])
+def test_encoder_kernel_on_nan_blocks_under_negative_moments(ext, signs):
+    """Negative importances (nothing forbids them) next to NaN and infinite weights: the torch operations' bytes."""
+    lut = hardware.device_palette("cuda").reshape(255, 255, 8)
+    weight, hdiag = matrix(12, 256, torch.float32, seed=6)
+    weight[3, 5] = float("nan")
+    weight[4, 9] = float("inf")
+    weight[5, 200] = float("-inf")
+    weight[6] = float("nan")
+    hdiag[:: 3 if signs == "some" else 1] *= -1
+    want_blocks, _ = torch_encode(weight, hdiag, lut)
+    assert torch.equal(encoder.encode_matrix_tensor(weight, hdiag, lut)[0], want_blocks)
+
+
 def test_encoder_takes_strided_offset_and_host_rows(ext):
     """What the torch operations accept: a transposed view, rows at an odd offset, float64, a CPU matrix in
     chunks; and encode_rows' chunks are the same bytes."""

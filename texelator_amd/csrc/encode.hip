@@ -146,7 +146,9 @@ __device__ __forceinline__ uint2 encode_one(const float (&v)[16], const float (&
 
   // 3. the 3 x 3 neighbourhood: weighted squared error, the first strict improvement wins. Only
   // the distance to the nearest value is needed here; the selectors are found once, at the end.
-  float best_error = INFINITY;
+  // A block that holds a NaN (hi is one) keeps its start, as every torch error of it is NaN: the minima
+  // below skip NaN, and negative importances would turn what they leave into an improvement.
+  float best_error = hi != hi ? -INFINITY : INFINITY;
 #pragma unroll 1
   for (int d0 = -1; d0 <= 1; ++d0) {
     const int c0 = min(max(center0 + d0, -127), 127);
