@@ -98,3 +98,13 @@ def test_encoder_takes_strided_offset_and_host_rows(ext):
     assert (blocks == want_blocks.cpu().numpy()).all() and (scales == want_scales.cpu().numpy()).all()
     with pytest.raises(_hip.TexelatorError):
         _hip.encode_bc4(weight, hdiag[:-1].contiguous(), lut)
+
+
+def test_tables_of_another_shape_are_refused(ext):
+    """A palette table must be [255, 255, 8]: the torch operations cannot index a flat one, with a GPU table either."""
+    lut = hardware.device_palette("cuda").reshape(255, 255, 8)
+    weight, hdiag = matrix(4, 64, torch.float32, seed=1)
+    with pytest.raises(IndexError):
+        encoder.encode_matrix_tensor(weight, hdiag, lut.reshape(-1))
+    with pytest.raises(IndexError):
+        encoder.encode_matrix(weight, hdiag, lut.reshape(-1))

@@ -16,6 +16,7 @@ from pathlib import Path
 import numpy as np
 import torch
 
+PALETTE_SHAPE = (255, 255, 8)
 PALETTE_FLOATS = 255 * 255 * 8
 
 
@@ -146,8 +147,8 @@ def pack_blocks_tensor(endpoint0: torch.Tensor, endpoint1: torch.Tensor, indices
 def _native_encode(lut: torch.Tensor, hdiag: torch.Tensor, k: int):
     """The library's encoder for row chunks of K columns on ``lut``'s GPU: a function of a chunk (any
     device, type or strides) giving ``(blocks, scales)`` device tensors; None where the torch
-    operations run (a CPU table, or a table or moments of another form)."""
-    if not (lut.is_cuda and lut.dtype == torch.float32 and lut.numel() == PALETTE_FLOATS and hdiag.numel() == k):
+    operations run (a CPU table, or a table or moments of another form, which they take or refuse)."""
+    if not (lut.is_cuda and lut.dtype == torch.float32 and tuple(lut.shape) == PALETTE_SHAPE and hdiag.numel() == k):
         return None
     from . import _hip
 
