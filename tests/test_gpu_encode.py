@@ -108,3 +108,21 @@ def test_tables_of_another_shape_are_refused(ext):
         encoder.encode_matrix_tensor(weight, hdiag, lut.reshape(-1))
     with pytest.raises(IndexError):
         encoder.encode_matrix(weight, hdiag, lut.reshape(-1))
+
+
+@pytest.mark.parametrize("form", ["transposed", "float64", "offset"])
+def test_matrices_that_must_be_copied_are_copied_in_chunks(ext, form):
+    """A matrix the kernel cannot read where it lies is staged rows_per_chunk rows at a time: the scratch stays a
+    fraction of the matrix, and the bytes are those of the matrix in place."""
+    lut = hardware.device_palette("cuda").reshape(255, 255, 8)
+    weight, hdiag = matrix(4096, 1024, torch.float32, seed=2)
+    want_blocks, want_scales = encoder.encode_matrix_tensor(weight, hdiag, lut)
+    view = {"transposed": lambda: weight.t().contiguous().t(), "float64": weight.double,
+            "offset": lambda: torch.nn.functional.pad(weight.reshape(-1), (1, 0))[1:].view(4096, 1024)}[form]()
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    blocks, scales = encoder.encode_matrix_tensor(view, hdiag, lut, rows_per_chunk=256)
+    scratch = torch.cuda.max_memory_allocated() - before - blocks.numel() - 4 * scales.numel()
+    assert scratch < weight.numel() * 4 // 4
+    assert torch.equal(blocks, want_blocks) and torch.equal(scales, want_scales)

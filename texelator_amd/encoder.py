@@ -144,6 +144,15 @@ def pack_blocks_tensor(endpoint0: torch.Tensor, endpoint1: torch.Tensor, indices
     return packed
 
 
+_KERNEL_DTYPES = (torch.float32, torch.bfloat16, torch.float16)
+
+
+def _read_in_place(weight: torch.Tensor, device: torch.device) -> bool:
+    """Whether the kernel reads ``weight`` where it lies; any other matrix is copied, a chunk at a time."""
+    return (weight.device == device and weight.dtype in _KERNEL_DTYPES and weight.is_contiguous()
+            and weight.data_ptr() % 16 == 0)
+
+
 def _native_encode(lut: torch.Tensor, hdiag: torch.Tensor, k: int):
     """The library's encoder for row chunks of K columns on ``lut``'s GPU: a function of a chunk (any
     device, type or strides) giving ``(blocks, scales)`` device tensors; None where the torch
@@ -155,8 +164,7 @@ def _native_encode(lut: torch.Tensor, hdiag: torch.Tensor, k: int):
     moments, table = hdiag.float().reshape(-1).contiguous(), lut.contiguous()
 
     def encode(rows: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
-        widened_there = rows.dtype in (torch.float32, torch.bfloat16, torch.float16)
-        rows = rows.detach().to(device=lut.device, dtype=rows.dtype if widened_there else torch.float32)
+        rows = rows.detach().to(device=lut.device, dtype=rows.dtype if rows.dtype in _KERNEL_DTYPES else torch.float32)
         return _hip.encode_bc4(rows.contiguous(), moments, table)
 
     return encode
@@ -172,8 +180,8 @@ def encode_matrix_tensor(weight: torch.Tensor, hdiag: torch.Tensor, lut: torch.T
         raise ValueError(f"unsupported K={k}; BC4 needs K % 16 == 0")
     hdiag = hdiag.to(lut.device)
     native = _native_encode(lut, hdiag, k)
-    if native is not None and weight.device == lut.device and 0 < m <= 0x7FFFFFFF and rows_per_chunk > 0:
-        return native(weight)  # resident: nothing to stage and no scratch, so one launch
+    if native is not None and _read_in_place(weight, lut.device) and 0 < m <= 0x7FFFFFFF and rows_per_chunk > 0:
+        return native(weight)  # nothing to stage and no scratch, so one launch
     blocks = torch.empty((m, k // 16 * 8), dtype=torch.uint8, device=lut.device)
     scales = torch.empty(m, dtype=torch.float32, device=lut.device)
     for start in range(0, m, rows_per_chunk):
