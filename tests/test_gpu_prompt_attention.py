@@ -63,6 +63,20 @@ def test_scores_that_grow_along_the_keys(ext, tokens, heads, scale):
     check(layers.prefill_attention(q, k, v, heads, heads, scale), reference(q, k, v, heads, scale))
 
 
+@pytest.mark.parametrize("tokens,heads,kv_heads", [(64, 8, 8), (512, 8, 1), (323, 28, 4), (704, 40, 8), (1409, 56, 7)])
+def test_a_token_does_not_reach_the_others(ext, tokens, heads, kv_heads):
+    """A query of far larger scores (its running maxima rise in other blocks) leaves the bits of every other query's
+    output, the earlier ones of its wave among them: under each split of the waves."""
+    q, k, v = inputs(tokens, heads, kv_heads, 11)
+    scale = 1 / math.sqrt(128)
+    want = layers.prefill_attention(q, k, v, heads, kv_heads, scale)
+    loud = 32 * (tokens // 32) - 1  # the last of the last whole group of 32 queries
+    q[loud] *= 30
+    got = layers.prefill_attention(q, k, v, heads, kv_heads, scale)
+    rows = [t for t in range(tokens) if t != loud]
+    assert torch.equal(got[rows], want[rows]) and not torch.equal(got[loud], want[loud])
+
+
 @pytest.mark.parametrize("tokens,heads", [(77, 4), (300, 40)])
 def test_caches_and_outputs_off_alignment(ext, tokens, heads):
     """Caches 2 bytes off a 16-byte boundary and output rows at odd strides give the aligned call's bits."""

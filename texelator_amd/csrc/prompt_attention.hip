@@ -18,17 +18,22 @@
 //     transpose is done by the read itself (ds_read_b64_tr_b16). The descriptors end at the last token:
 //     rows past it read as zeros, so stale cache rows never reach a sum;
 //   * one barrier per key block.
-// Online softmax in fp32 with exp2 (reference exponent m and sum l per query). Probabilities are rounded
+// Online softmax in fp32 with exp2 (running maximum m and sum l per query). Probabilities are rounded
 // to bf16 and their rounded values are what l sums.
 //
-// Bound: a wave's block costs ~2900 cycles at one or two waves per SIMD: 32 products (1024 matrix
-// cycles), ~240 VALU instructions (32 of them exponentials, 4 issue slots each) and 32 KiB of LDS operand
-// reads, none dominant (copies without the staging, the exponentials, either product or either operand
-// read were each 4-20% faster). Measured and no better: the next block's score products woven into this
-// block's exponentials and its scaling into the value products by hand (32.0 against 31.8 us at 1000
-// tokens and 40/8 heads with <4, 1>). Kernel this replaced (16x16x32 products, 16 queries per wave, probabilities
-// through LDS, three barriers per key block, values transposed by the stores): 73.8 us at 1000 tokens and
-// 40/8 heads, 641.8 us at 4096; this one 27.1 and 209 us.
+// Bound: the chain of key blocks of the last queries. By the slope over 1000 to 1536 tokens at 16/2 heads a block of 64
+// keys takes a wave alone on its SIMD 1.42 us, two waves of a SIMD 2.24 us for a block each; the launch, the first
+// block's loads and the end take 4 us (<4, 1>) to 6 (<4, 2>, with its merge). A block is 32 products (1024
+// matrix cycles), ~300 VALU instructions (32 of them exponentials, 4 issue slots each) and 32 KiB of LDS operand
+// reads, none dominant (copies without the staging, the exponentials, either product or either operand read were
+// each 4-20% faster). At 1000 tokens and 40/8 heads <4, 2> has 320 workgroups, one a CU (LDS): eight turns and
+// the fixed 6 us are 24 of its 25.1 us. Measured and level: the next block's score products woven into this block's
+// exponentials, and its scaling into the value products, by hand. Letting the maximum lag until it has grown by
+// 2^8 saved most rescaling (62.7 against 67.7 us at 2048 tokens and 40/8 heads, 27.1 against 27.6 at 1000), but
+// tied a query's rounding to the others of its wave and raised the error against 64 bits (2.06e-3 against 2.01e-3).
+// Kernel this replaced (16x16x32 products, 16 queries per wave, probabilities through LDS, three barriers per key
+// block, values transposed by the stores), launches back to back: 72.9 us at 1000 tokens and 40/8 heads, 210 at
+// 2048, 314 at 4096 and 16/2 heads; this one 27.6, 67.7 and 99.
 #include <math.h>
 
 #include <type_traits>
@@ -65,8 +70,9 @@ __device__ __forceinline__ float halves_sum(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Two waves per SIMD, but for <1, 4, 32>, whose four waves hold all of a CU's LDS.
 template <int QW, int KW, int KB>
-__global__ __launch_bounds__(64 * QW * KW, 2) __attribute__((amdgpu_num_vgpr(256))) void prompt_attention_kernel(
+__global__ __launch_bounds__(64 * QW * KW, QW * KW * KB == 128 ? 1 : 2) __attribute__((amdgpu_num_vgpr(256))) void prompt_attention_kernel(
     const uint16_t *q, int64_t q_stride, const uint16_t *k_cache, const uint16_t *v_cache, int tokens, int heads,
     int group, int64_t max_ctx, float scale, uint16_t *out, int64_t out_stride, int direct) {
   constexpr int kTile = KB * kRowBytes;  // bytes of a key (or value) block
@@ -181,13 +187,11 @@ __global__ __launch_bounds__(64 * QW * KW, 2) __attribute__((amdgpu_num_vgpr(256
     for (int s = 0; s < NS; ++s)
 #pragma unroll
       for (int r = s == 0 ? 2 : 0; r < 16; r += 2) mx = fmaxf(fmaxf(mx, sc[s][r]), sc[s][r + 1]);
-    // The reference exponent m follows the running maximum only when that has grown by more than
-    // kGrow: probabilities then reach 2^kGrow instead of 1 (the same relative precision in bf16 and
-    // fp32), and O is seldom rescaled. (Finite: every query has a key <= itself in every block it reaches.)
-    constexpr float kGrow = 8.f;
-    const float top = halves_max(mx);
-    if (__builtin_amdgcn_ballot_w64(top > m + kGrow) != 0) {
-      const float mnew = fmaxf(m, top);
+    // The running maximum is each query's own: a query that finds no larger score scales by exactly 1, so
+    // its output does not depend on which other queries share the wave. (m is finite from a query's first block
+    // on, where its scores are: every query has a key <= itself in every block it reaches.)
+    const float mnew = fmaxf(m, halves_max(mx));
+    if (__builtin_amdgcn_ballot_w64(mnew > m) != 0) {
       const float alpha = __builtin_amdgcn_exp2f(m - mnew);
       l *= alpha;
 #pragma unroll
@@ -341,14 +345,14 @@ hipError_t launch_prefill_attention(const uint16_t *q, int64_t q_stride, const u
                        stream, q, q_stride, k_cache, v_cache, (int)tokens, heads, heads / kv_heads, max_ctx, scale, out, out_stride, direct);
   };
   // Which split of the waves: by how many workgroups of 128, 64 and 32 queries there are. Measured at
-  // 17 .. 4096 tokens and 40/8, 28/4 and 16/2 heads (us):
-  //   <4, 1> from 2.25 workgroups of 128 queries a CU (two are resident): 2048 tokens, 40 heads 67 against 79
-  //          of <4, 2> (1.75 to 2 of them: 57-104 against 60-114); and for up to 64 tokens, where there is no
-  //          chain to shorten (4.8 against 6.2-7.2);
-  //   <4, 2> from 1.6 workgroups of 64 queries a CU: 1000 tokens, 40 heads 27.1 against 30.6 of <4, 1> and
-  //          37.2 of <2, 4>;
-  //   <1, 4> while workgroups of 32 queries fit the CUs at once: 512 tokens, 16 heads 11.1 against 12.3 of
-  //          <2, 4> and 14.8 of <4, 1>; <2, 4> between: 1000 tokens, 16 heads 18.7 against 23.4-26.2.
+  // 17 .. 4096 tokens and 40/8, 32/8, 28/4 and 16/2 heads (us, graph replays):
+  //   <4, 1> from 2.25 workgroups of 128 queries a CU (two are resident): 2048 tokens, 40 heads 61.6 against 71.9
+  //          of <4, 2> (at 1.7 to 2 of them 37.0 - 57.3 against 37.9 - 52.3); and for up to 64 tokens, where there
+  //          is no chain to shorten (4.2 - 5.0 against 5.7 - 7.4);
+  //   <4, 2> from 1.6 workgroups of 64 queries a CU: 1000 tokens, 40 heads 25.1 against 29.3 of <4, 1> and
+  //          35.6 of <2, 4>;
+  //   <1, 4> while workgroups of 32 queries fit the CUs at once: 512 tokens, 16 heads 12.0 against 12.8 of
+  //          <2, 4> and 15.5 of <4, 1>; <2, 4> between: 1000 tokens, 16 heads 18.7 against 24.0 - 26.7.
   const int64_t tiles128 = (tokens + 127) / 128 * heads, tiles64 = (tokens + 63) / 64 * heads,
                 tiles32 = (tokens + 31) / 32 * heads;
   if (tokens <= 64 || 4 * tiles128 >= 9 * (int64_t)cus) launch(prompt_attention_kernel<4, 1, 64>, 128, 4);
