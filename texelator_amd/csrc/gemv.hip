@@ -14,7 +14,8 @@
 //     the partials in split order, so results never depend on scheduling; where the row groups
 //     spread evenly over the CUs, one workgroup instead runs every split of its row group and sums
 //     them in the same order (gemv_fused_kernel: the same bits, one launch).
-// Single-token calls stage x in LDS; multi-token calls read x through the cache hierarchy.
+// Single-token calls stage x in LDS; multi-token calls read x through the cache hierarchy, or split K with
+// the activations in LDS (gemv_batch_kernel).
 #include <algorithm>
 
 #include "bc4_device.h"
@@ -551,9 +552,9 @@ __global__ __launch_bounds__(kThreads, LUT || XSRC != kXRead ? 4 : TX_GEMV_WAVES
   }
 }
 
-// Several tokens (2 to 16) through one pass of the weights where K is long (gemv_batch_splits), K split so that the chip is full whatever the
-// matrix's shape: a workgroup of eight waves takes eight row groups (one per wave) x one K range, with
-// the range's activations of all tokens in LDS, and writes fp32 partials [split][token][Mp] that
+// Several tokens (2 to 16) through one pass of the weights where a split of K pays (gemv_batch_splits), so that the
+// chip is full whatever the matrix's shape: a workgroup of eight waves takes eight row groups (one per wave) x one K
+// range, with the range's activations of all tokens in LDS, and writes fp32 partials [split][token][Mp] that
 // splitk_reduce_kernel sums in split order. Each wave streams the whole range of its own row group, so
 // nothing crosses waves and the K loop has no barrier.
 //   * What bounds it is the decode, as in the one-token kernel; gemv_kernel<MULTI> instead read every
@@ -987,16 +988,34 @@ bool gemv_fused_profitable(int RG, int CG, int ks, int cus) {
 }
 
 int gemv_batch_splits(int RG, int CG, int K, int64_t tokens, int cus) {
-  // From 4097 input features: below, the unsplit kernel's four waves a row group have few tiles each and
-  // the reduce launch costs more than it gains (us, unsplit against split: 2048 x 2048 at 8 tokens 5.5 / 5.9,
-  // 11008 x 2048 at 15 9.3 / 10.9; 1024 x 5120 at 8 9.0 / 7.5, 27648 x 5120 at 2 22.2 / 22.3 and at 15
-  // 46.0 / 28.5, 5120 x 27648 at 8 46.6 / 25.7).
   if (tokens < 2 || tokens > 16 || CG <= 32 || tokens * K > 0x3FFFFFF0) return 0;
+  // Where the split and its second launch (~1.3 us of host time, and the reduce) pay. Unsplit, a wave's chain
+  // is a quarter of K, and every tile reads all tokens' activations: so for long K (less long where more rows
+  // keep the reduce small beside the chain), or for much work. us a call, unsplit against split, launches replayed as
+  // a graph / from Python:
+  //   long K: 1024 x 8192 at 8 tokens 12.5 / 12.6 against 9.2 / 11.9, 64 x 11008 at 5 14.8 / 14.9 against 10.8 / 12.3,
+  //   5120 x 7168 at 5 13.4 / 13.5 against 10.7 / 12.4, 5120 x 27648 at 8 47.0 / 47.1 against 23.8 / 24.1; below the
+  //   lines 256 x 8192 at 5 11.3 / 11.6 against 10.0 / 12.2, 4096 x 7168 at 4 11.4 / 11.7 against 9.8 / 12.2, 5120 x
+  //   6144 at 5 11.7 / 11.8 against 10.0 / 12.4, 64 x 4112 at 4 5.9 / 10.8 against 7.1 / 12.3;
+  //   much work: 27648 x 5120 at 8 31.9 against 23.5, 11008 x 5120 at 12 16.3 against 13.9 (0.68e9); below
+  //   17408 x 4112 at 8 14.8 against 15.0 (0.57e9), 7168 x 4112 at 15 9.8 against 11.5 (0.44e9).
+  const bool long_chain = CG >= 80 || (CG >= 64 && RG >= 64) || (CG >= 56 && RG >= 320);
+  const bool much_work = tokens * K * RG * kTileRows >= 600000000;
+  if (!long_chain && !much_work) return 0;
   // About twelve waves a CU (16 to 32 were level to 25% slower: more partials); at most as many splits
   // as keep the partials a quarter of the weights' bytes (ks * tokens * 4 against K / 2 / 4 per row);
   // at least as many as the LDS needs.
-  const int waves = (RG + kBatchWaves - 1) / kBatchWaves * kBatchWaves;
-  int ks = (12 * cus + waves - 1) / waves;
+  const int groups = (RG + kBatchWaves - 1) / kBatchWaves;  // workgroups a split
+  int ks = (12 * cus + groups * kBatchWaves - 1) / (groups * kBatchWaves);
+  // With up to three splits a round of the CUs more or less shows: where the fullest CU has at least a third more
+  // than its share, the best of this count and the next two. Before and now: 22016 x 5120 at 15 tokens (3 -> 4 splits, 516
+  // -> 688 workgroups) 26.1 -> 22.1 us, 22016 x 4112 at 8 19.3 -> 18.2 (unsplit 18.2).
+  auto rounds = [&](int s) { return (int64_t)((groups * (int64_t)s + cus - 1) / cus); };
+  if (ks <= 3 && 3 * rounds(ks) * cus >= 4 * (int64_t)groups * ks) {
+    const int first = ks;
+    for (int s = first + 1; s <= first + 2; ++s)
+      if (rounds(s) * ks < rounds(ks) * s) ks = s;
+  }
   ks = std::min(ks, std::max(1, (int)(K / (32 * tokens))));
   const int max_cols = kBatchLdsBytes / (int)((tokens + 3) / 4 * 1024);
   ks = std::min(std::max(ks, (CG + max_cols - 1) / max_cols), CG);
