@@ -69,9 +69,11 @@ int tx_concat_rows(const uint64_t *handles, int count, uint64_t *handle_out);
  *             aligned (may be NULL when that is 0), stream-ordered: the prefill path's split-K
  *             partials or backend 1's dense rows (required), or a one-token GEMV's split-K partials (optional: with NULL the
  *             handle's own buffer is used, so two such calls on one handle must not overlap), or
- *             the batched GEMV's for a few tokens (optional: see tx_linear_workspace_bytes)
+ *             the batched GEMV's for 2 to 16 tokens below the prefill threshold (optional: without it, or
+ *             with less than tx_linear_workspace_bytes, the call runs unsplit, with sums in another order)
  * tokens >= prefill threshold (and tokens > 1) uses the prefill GEMM candidate set by
- * tx_set_prefill_backend; otherwise the decode GEMV with the configured lookahead.
+ * tx_set_prefill_backend; otherwise the decode GEMV with the configured lookahead (the batched GEMV has
+ * a fixed one; the lookahead never changes a result).
  * The reference allocates its prefill scratch inside the call (texelator_cuda.cu:942-957); here
  * the caller supplies it, so the library never allocates on this path. */
 int tx_linear(uint64_t handle, const void *x, int x_dtype, int64_t x_numel, int64_t x_last,
@@ -79,8 +81,9 @@ int tx_linear(uint64_t handle, const void *x, int x_dtype, int64_t x_numel, int6
 
 /* tx_linear for callers that cannot allocate (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc). No counterpart in the reference. Same arguments, dispatch,
- * checks and results (bit for bit) as tx_linear, but there is no workspace argument and the
- * handle's own split-K buffer is not used: split-K partial sums go to a static 32 MiB device
+ * checks and results (bit for bit) as tx_linear with the workspace of tx_workspace_bytes, but there is
+ * no workspace argument and the handle's own split-K buffer is not used: the split-K partial sums of every
+ * kind of call (one token, a few tokens, prefill) go to a static 32 MiB device
  * array of the library (tx_noalloc_scratch_bytes), one per GPU, kept until the process ends.
  * No hipMalloc, hipFree or allocating library call is made. A call whose partials would exceed
  * the array fails with TX_ERR_INVALID before launching anything; a prefill-sized call on a handle
@@ -117,7 +120,8 @@ int tx_fp4_gemm(const uint8_t *x_packed, const uint8_t *x_scales, const uint8_t 
 int tx_noalloc_scratch_bytes(int64_t *bytes);
 
 /* Workspace bytes of tx_linear and tx_prefill for `tokens` tokens: the prefill split-K partial
- * sums for tokens > 1 (with backend 1 and tokens >= the prefill threshold: the dense scratch of
+ * sums for tokens > 1, or the batched GEMV's for 2 to 16 tokens below the prefill threshold if those
+ * are more (with backend 1 and tokens >= the prefill threshold: the dense scratch of
  * min(tile_rows, M) decoded rows of K 16-bit weights rounded up to 256 bytes, 256 bytes of slack
  * and 8 MiB for the library GEMM, whose workspace starts at the first 256-byte boundary after the
  * rows; the caller's workspace need only be 16-byte aligned), the one-token GEMV's split-K partials for
@@ -126,10 +130,10 @@ int tx_noalloc_scratch_bytes(int64_t *bytes);
  * reference counterpart (see tx_linear). */
 int tx_workspace_bytes(uint64_t handle, int64_t tokens, int64_t *bytes);
 
-/* Workspace bytes tx_linear itself can use for `tokens` tokens: tx_workspace_bytes for one token and at or
- * above the prefill threshold; for several tokens below it the K-split partials of the batched GEMV
- * (2 to 16 tokens; 0 where it does not run). There the workspace is optional: without one of this size
- * tx_linear runs that call unsplit, slower, with sums in another order. */
+/* Workspace bytes tx_linear itself uses for `tokens` tokens, at most tx_workspace_bytes: the same for one token
+ * and at or above the prefill threshold; for several tokens below it only the K-split partials of the
+ * batched GEMV (2 to 16 tokens; 0 where it does not run). There the workspace is optional: without one of
+ * this size tx_linear runs that call unsplit, slower, with sums in another order. */
 int tx_linear_workspace_bytes(uint64_t handle, int64_t tokens, int64_t *bytes);
 
 /* Decode GEMV with float32 output and no bias, for parity checks (no reference counterpart:

@@ -74,7 +74,7 @@ def test_tokens_do_not_reach_each_other(ext, k):
         ext.free(handle)
 
 
-def unsplit(handle, x, y, workspace=None):
+def linear_with(handle, x, y, workspace=None):
     """tx_linear with the given workspace address and size (none by default)."""
     address, size = workspace or (None, 0)
     status = _lib.load().tx_linear(handle, ctypes.c_void_p(x.data_ptr()), _lib.TX_DTYPE_BF16, x.numel(), x.shape[-1], 0,
@@ -96,12 +96,28 @@ def test_without_a_workspace_the_call_runs_unsplit(ext):
         ext.linear_noalloc_into(handle, x, y)
         assert torch.equal(y, want)
         plain = torch.empty_like(want)
-        unsplit(handle, x, plain)
+        linear_with(handle, x, plain)
         assert torch.allclose(plain.float(), want.float(), rtol=2 ** -7, atol=1e-2)
         scratch = torch.full((need + 16,), 0x55, dtype=torch.uint8, device="cuda")
         for workspace in ((scratch.data_ptr(), need - 1), (scratch.data_ptr() + 8, need)):
-            unsplit(handle, x, y, workspace)
+            linear_with(handle, x, y, workspace)
             assert torch.equal(y, plain) and bool((scratch == 0x55).all())
+    finally:
+        ext.free(handle)
+
+
+@pytest.mark.parametrize("m,k,tokens", [(96, 10240, 5), (1024, 8192, 15), (22016, 4224, 8), (11008, 5120, 13), (64, 4112, 7)])
+def test_the_documented_workspace_gives_the_static_scratch_entry_points_bits(ext, m, k, tokens):
+    """tx_linear with a workspace of tx_workspace_bytes, as a C caller allocates it, and tx_linear_noalloc."""
+    handle, _, _ = pack(ext, m, k, 19)
+    try:
+        x = bf16_vector((tokens, k), 20).cuda()
+        y, want = (torch.empty((tokens, m), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        scratch = torch.empty(max(16, ext.workspace_bytes(handle, tokens)), dtype=torch.uint8, device="cuda")
+        assert split_bytes(handle, tokens) <= ext.workspace_bytes(handle, tokens)
+        linear_with(handle, x, y, (scratch.data_ptr(), ext.workspace_bytes(handle, tokens)))
+        ext.linear_noalloc_into(handle, x, want)
+        assert torch.equal(y, want) and torch.equal(ext.linear(handle, x), want)
     finally:
         ext.free(handle)
 
@@ -126,7 +142,7 @@ def test_sides_of_the_splits_lines(ext, m, k, tokens, split):
         x = bf16_vector((tokens, k), 18).cuda()
         got = ext.linear(handle, x)
         want = torch.empty_like(got)
-        unsplit(handle, x, want)
+        linear_with(handle, x, want)
         if split:
             error = (got.float() - want.float()).abs()
             assert bool((error <= 2 ** -7 * want.float().abs() + 1e-3 * want.float().square().mean().sqrt()).all())

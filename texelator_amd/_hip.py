@@ -53,7 +53,7 @@ def _aligned(x: torch.Tensor) -> torch.Tensor:
 
 
 def workspace_bytes(handle: int, tokens: int) -> int:
-    """Device scratch the prefill path needs for ``tokens`` tokens (``tx_workspace_bytes``)."""
+    """Device scratch that covers every call of ``tokens`` tokens (``tx_workspace_bytes``)."""
     out = ctypes.c_int64(0)
     check(_lib.load().tx_workspace_bytes(handle, int(tokens), ctypes.byref(out)))
     return int(out.value)

@@ -223,8 +223,9 @@ tx::SplitSource split_source(const Handle *h) {
   return tx::SplitSource{h->partials, static_cast<const uint16_t *>(h->bias), h->gemv_splits, h->Mp, 1};
 }
 
-// One-token K splits write ks * Mp fp32 partials to `partials` (the handle's own buffer, or the
-// static scratch of tx_linear_noalloc); several tokens run unsplit and write none.
+// One-token K splits write ks * Mp fp32 partials to a caller's workspace, the handle's own buffer or the
+// static scratch of tx_linear_noalloc; several tokens below the prefill threshold write theirs, where they
+// are split (batch_partials_bytes), to a workspace or that scratch.
 // One-token calls of this handle run every K split in one workgroup (gemv_fused_kernel).
 bool one_token_fused(const Handle *h) {
   return !h->lut && tx::gemv_fused_profitable(h->RG, h->CG, h->gemv_splits, h->cus);
@@ -682,7 +683,8 @@ int tx_workspace_bytes(uint64_t value, int64_t tokens, int64_t *bytes) {
   if (!h) return fail(TX_ERR_INVALID, "null Texelator handle");
   if (!bytes) return fail(TX_ERR_INVALID, "null output");
   if (tokens > 1 && tokens >= h->prefill_threshold) *bytes = prefill_call_bytes(h, tokens);
-  else *bytes = tokens > 1 ? prefill_workspace_bytes(h, tokens) : gemv_partials_bytes(h, tokens);
+  else if (tokens > 1) *bytes = std::max(prefill_workspace_bytes(h, tokens), batch_partials_bytes(h, tokens));
+  else *bytes = gemv_partials_bytes(h, tokens);
   return TX_OK;
 }
 
