@@ -413,6 +413,15 @@ int tx_rope_kv_cache_split(uint64_t qkv_handle, const int64_t *positions, const 
 int tx_prefill_split(uint64_t handle, const void *x, int64_t tokens, void *workspace, int64_t workspace_bytes,
                      int *splits, void *stream);
 
+/* The faster path for a call of `tokens` tokens whose output a prefill split consumer can take: whole (K is not split,
+ * the call is below the prefill threshold or runs backend 1: tx_prefill_split refuses it), partials
+ * (tx_prefill_split and the consumer), or summed (tx_linear, whose tile sums its splits itself, and the plain
+ * helper; tx_prefill_split runs as well). The bits are the same on every path. */
+#define TX_PREFILL_WHOLE 0
+#define TX_PREFILL_PARTIALS 1
+#define TX_PREFILL_SUMMED 2
+int tx_prefill_plan(uint64_t handle, int64_t tokens, int *plan);
+
 /* tx_add_rmsnorm for `tokens` rows whose delta is tx_linear's output of delta_handle (M ==
  * hidden), read from the partials tx_prefill_split left: summed in split order and rounded as the
  * prefill reduce does (the bias added with a second rounding), bit for bit. */

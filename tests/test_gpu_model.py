@@ -353,6 +353,26 @@ def test_rope_kv_cache_prefill_split_is_bit_identical(ext, heads, kv, k, tokens)
         ext.free(handle)
 
 
+@pytest.mark.parametrize("m,k,tokens,plan", [
+    (64, 1920, 40, "WHOLE"), (2048, 2048, 15, "WHOLE"), (2048, 2048, 16, "SUMMED"), (2048, 2048, 128, "SUMMED"),
+    (2048, 2048, 129, "PARTIALS"), (7168, 5120, 96, "SUMMED"), (7168, 5120, 97, "PARTIALS"), (2048, 11008, 64, "PARTIALS"),
+    (16384, 4096, 64, "SUMMED")])
+def test_prefill_plan(ext, m, k, tokens, plan):
+    """Both sides of the plan's lines; every path it names gives linear's bits."""
+    handle = _random_handle(ext, m, k, seed=m)
+    try:
+        assert layers.prefill_plan(handle, tokens) == getattr(_lib, "TX_PREFILL_" + plan)
+        x = torch.randn(tokens, k, device="cuda", generator=torch.Generator(device="cuda").manual_seed(k)).bfloat16()
+        ws, want = _prefill_workspace(ext, handle, tokens), ext.linear(handle, x)
+        assert torch.equal(layers.linear_into(handle, x, torch.empty_like(want), ws), want)
+        if plan != "WHOLE":
+            assert layers.prefill_split(handle, x, ws) > 1
+        with pytest.raises(_lib.TexelatorError):
+            layers.linear_into(handle, x, want[1:], ws)
+    finally:
+        ext.free(handle)
+
+
 def test_prefill_split_refusals(ext):
     """prefill_split runs nothing where its call would not split K (a 512-token gate GEMM on the
     wide tile), below the prefill threshold, or on the dense backend: UnsupportedError."""
@@ -391,6 +411,31 @@ def test_decoder_prefill_with_split_consumers_is_bit_identical(ext, config):
             plain = model.hidden_states(ids, positions, 512)
         assert torch.equal(split, plain)
         assert torch.equal(kc, model.k_cache) and torch.equal(vc, model.v_cache)
+    finally:
+        model.close()
+
+
+@pytest.mark.parametrize("tokens,split", [(20, {"down"}), (77, {"down"}), (128, {"down"}), (200, {"qkv", "o", "down"})])
+def test_short_prompts_run_the_tile_that_sums_its_splits(ext, monkeypatch, tokens, split):
+    """A 3B-class layer: where linear's default is the split-group tile (q|k|v and o up to 128 tokens) the prompt takes
+    it, elsewhere the partials go to the consumer; the hidden states are the plain path's either way, bit for bit."""
+    from dataclasses import replace
+
+    model = modeling.BC4Decoder(replace(modeling.DecoderConfig.qwen25_3b_style(), layers=1), max_context=256, seed=7)
+    names = {handle: key for key, handle in model.layers[0].handles.items()}
+    calls = []
+    prefill_split = layers.prefill_split
+    monkeypatch.setattr(layers, "prefill_split", lambda handle, *rest: calls.append(names[handle]) or prefill_split(handle, *rest))
+    try:
+        ids = prefill.prompt_ids(model, tokens)
+        positions = model.key_positions[:tokens]
+        with torch.inference_mode():
+            got = model.hidden_states(ids, positions, tokens).clone()
+            assert set(calls) == split
+            model.split_prefill = False
+            assert torch.equal(got, model.hidden_states(ids, positions, tokens))
+        plans = {True: _lib.TX_PREFILL_PARTIALS, False: _lib.TX_PREFILL_SUMMED}
+        assert all(layers.prefill_plan(h, tokens) == plans[key in split] for h, key in names.items() if key != "gate_up")
     finally:
         model.close()
 

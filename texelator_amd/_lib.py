@@ -22,6 +22,7 @@ TX_ERR_UNSUPPORTED = 3
 TX_DTYPE_F16 = 0
 TX_DTYPE_BF16 = 1
 TX_DTYPE_F32 = 2
+TX_PREFILL_WHOLE, TX_PREFILL_PARTIALS, TX_PREFILL_SUMMED = 0, 1, 2
 
 # name -> (restype, argtypes); every symbol declared in include/texelator_hip.h
 _P = ctypes.c_void_p
@@ -80,6 +81,7 @@ SIGNATURES = {
     "tx_linear_swiglu_norm": (_I32, [_U64, _P, _P, _U64, _P, ctypes.c_float, _P, _P]),
     "tx_linear_split_embed_norm": (_I32, [_U64, _P, _I64, _P, _P, _P, ctypes.c_float, _P]),
     "tx_rope_kv_cache_split": (_I32, [_U64, _P, _P, _P, _I32, _I32, _I32, _P, _P, _P, _I64, _P]),
+    "tx_prefill_plan": (_I32, [_U64, _I64, ctypes.POINTER(ctypes.c_int)]),
     "tx_prefill_split": (_I32, [_U64, _P, _I64, _P, _I64, ctypes.POINTER(ctypes.c_int), _P]),
     "tx_add_rmsnorm_prefill_split": (_I32, [_P, _U64, _P, _I64, _P, ctypes.c_float, _P, _I64, _P]),
     "tx_rope_kv_cache_prefill_split": (_I32, [_U64, _P, _I64, _P, _P, _P, _I32, _I32, _I32, _P, _P, _P, _I64, _P]),

@@ -980,6 +980,19 @@ tx::SplitSource prefill_split_source(const Handle *h, const void *partials, int6
                          tx::prefill_splits(h->M, h->K, tokens, h->cus), h->Mp, (int)tokens, 1};
 }
 
+int tx_prefill_plan(uint64_t value, int64_t tokens, int *plan) {
+  g_last_error.clear();
+  Handle *h = as_handle(value);
+  if (!h) return fail(TX_ERR_INVALID, "null Texelator handle");
+  if (!plan) return fail(TX_ERR_INVALID, "null output");
+  *plan = TX_PREFILL_WHOLE;
+  if (tokens < 2 || tokens < h->prefill_threshold || tokens > (1 << 20)) return TX_OK;
+  const int candidate = prefill_choice(h, tokens), ks = tx::prefill_splits(h->M, h->K, tokens, h->cus);
+  if (candidate == kDenseBackend || ks == 1) return TX_OK;
+  *plan = tx::prefill_partials_pay(candidate, h->M, h->K, tokens, ks, h->cus) ? TX_PREFILL_PARTIALS : TX_PREFILL_SUMMED;
+  return TX_OK;
+}
+
 int tx_prefill_split(uint64_t value, const void *x, int64_t tokens, void *workspace, int64_t workspace_bytes,
                      int *splits_out, void *stream) {
   g_last_error.clear();

@@ -1793,7 +1793,7 @@ void launch_wave_as(const PrefillParams &p, hipStream_t stream) {
 // caller): no reduce launch. Elsewhere the register-decoding 32-token tile, which was faster with
 // split partials (down 27648 -> 5120 at 32 tokens: 40.1 vs 42.0 us). Both give the same bits.
 hipError_t launch_small(const PrefillParams &p, hipStream_t stream) {
-  if (!TX_SMALL_WAVE || p.ks != 4 || p.tokens > kWaveMaxTokens || p.K % kTileK != 0 || p.no_reduce)
+  if (!prefill_sums_splits(9, p.K, p.tokens, p.ks) || p.no_reduce)
     return launch_tile<1, 1, TX_PREFILL_LA_PLAIN, false>(p, stream);
   if (p.lut) {
     if (p.f16) launch_wave_as<true, true>(p, stream);
@@ -1918,6 +1918,21 @@ int prefill_splits(int M, int K, int64_t tokens, int cus) {
 int prefill_default_candidate(int M, int K, int64_t tokens, int cus) {
   if (tokens <= kWaveMaxTokens && wave_tile_pays(M, K, tokens, cus) && prefill_splits(M, K, tokens, cus) == 4) return 9;
   return prefill_register_candidate(M, K, tokens, cus);
+}
+
+bool prefill_sums_splits(int candidate, int K, int64_t tokens, int ks) {
+  return TX_SMALL_WAVE && candidate == 9 && ks == 4 && tokens <= kWaveMaxTokens && K % kTileK == 0;
+}
+
+bool prefill_partials_pay(int candidate, int M, int K, int64_t tokens, int ks, int cus) {
+  if (!prefill_sums_splits(candidate, K, tokens, ks)) return true;
+  // With a consumer that reads the partials (no reduce launch) against the split-group tile and the plain consumer: the
+  // tile is faster up to 64 tokens (4096 x 4096 at 20 14.9 / 11.8 us, 12288 x 5120 at 64 30.6 / 31.6) and in one round
+  // of the CUs (8192 x 3072 at 96 23.4 / 17.9); in two the partials are (7168 x 5120 at 97 26.7 / 30.2 and at 128
+  // 29.1 / 30.7, 8192 x 8192 at 128 36.8 / 39.4).
+  const int row_blocks = (M + 31) / 32, token_tiles = (int)((tokens + 31) / 32);
+  const int tbw = wave_token_blocks(row_blocks, token_tiles, cus);
+  return token_tiles > 2 && row_blocks * ((token_tiles + tbw - 1) / tbw) > cus;
 }
 
 bool prefill_candidate_eligible(int candidate, int M, int K) {
