@@ -415,8 +415,8 @@ int tx_prefill_split(uint64_t handle, const void *x, int64_t tokens, void *works
 
 /* The faster path for a call of `tokens` tokens whose output a prefill split consumer can take: whole (K is not split,
  * the call is below the prefill threshold or runs backend 1: tx_prefill_split refuses it), partials
- * (tx_prefill_split and the consumer), or summed (tx_linear, whose tile sums its splits itself, and the plain
- * helper; tx_prefill_split runs as well). The bits are the same on every path. */
+ * (tx_prefill_split and the consumer), or summed (tx_linear, whose tile or reduce kernel sums the splits, and the
+ * plain helper; tx_prefill_split runs as well). The bits are the same on every path. */
 #define TX_PREFILL_WHOLE 0
 #define TX_PREFILL_PARTIALS 1
 #define TX_PREFILL_SUMMED 2

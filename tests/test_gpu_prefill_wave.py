@@ -73,6 +73,16 @@ def test_k_that_was_whole_stays_whole(ext):
         ext.free(handle)
 
 
+@pytest.mark.parametrize("m,k,tokens,ks", [(3000, 4848, 128, 9), (3000, 4848, 129, 4), (1536, 8960, 200, 8),
+                                           (2560, 2048, 200, 4), (2048, 11008, 128, 16), (2048, 11008, 129, 10)])
+def test_finer_splits_past_128_tokens_only_where_they_double(ext, m, k, tokens, ks):
+    handle = pack(ext, m, k, "bf16")[0]
+    try:
+        assert splits(ext, handle, m, tokens) == ks
+    finally:
+        ext.free(handle)
+
+
 @pytest.mark.parametrize("tokens", [256, 257, 384, 385, 513, 640, 767, 768])
 @pytest.mark.parametrize("m,mode", [(3072, "bf16"), (3000, "f16_bias")])
 def test_sides_of_the_large_tiles_padding_rule(ext, oracle_threads, m, mode, tokens):

@@ -122,7 +122,7 @@ int prefill_splits(int M, int K, int64_t tokens, int cus);
 // Whether a call of `tokens` tokens with `ks` splits sums them inside the tile `candidate` (the split-group form: no
 // partials, no reduce launch) unless its partials are asked for.
 bool prefill_sums_splits(int candidate, int K, int64_t tokens, int ks);
-// Whether such a call with ks > 1 is faster with its partials left to a consumer (tx_prefill_split) than summed.
+// Whether a call with ks > 1 is faster with its partials left to a consumer (tx_prefill_split) than summed.
 bool prefill_partials_pay(int candidate, int M, int K, int64_t tokens, int ks, int cus);
 hipError_t launch_prefill(const PrefillParams &p, int candidate, hipStream_t stream);
 // Tile `candidate` (6-9) on a merged [gate | up] matrix (p.M = 2 * inter, inter a multiple of 16,

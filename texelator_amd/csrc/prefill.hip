@@ -1905,8 +1905,11 @@ int prefill_splits(int M, int K, int64_t tokens, int cus) {
   const int64_t coarse = std::max(1, CG / 8);
   // Below 256 tokens a grid that leaves CUs idle is split down to 4 columns, to one workgroup a CU (more, and
   // from 256 tokens any, cost as much in partials: level or slower). 2048 x 2048 at 16 tokens 12.5 -> 6.7 us,
-  // 1024 x 5120 at 16 12.6 -> 9.5, 3000 x 4848 at 77 20.2 -> 17.9. A K that was not split stays whole.
-  const int64_t fine = tokens < 256 && coarse > 1 ? std::min<int64_t>(CG / 4, cus / items) : 1;
+  // 1024 x 5120 at 16 12.6 -> 9.5, 3000 x 4848 at 77 20.2 -> 17.9. Past 128 tokens only to at least twice the
+  // splits: 3000 x 4848 at 200 tokens 24.5 us with four splits and a consumer of their partials, 25.2 with five;
+  // 1536 x 8960 at 255 26.7 with eight, 27.4 with ten. A K that was not split stays whole.
+  int64_t fine = tokens < 256 && coarse > 1 ? std::min<int64_t>(CG / 4, cus / items) : 1;
+  if (tokens > 128 && fine < 2 * coarse) fine = 1;
   ks = std::min(ks, std::max(coarse, fine));
   if (ks > 1 && wave_tile_pays(M, K, tokens, cus)) ks = 4;
   const int64_t cap = std::max<int64_t>(1, (int64_t(32) << 20) / (tokens * (int64_t)((M + 15) / 16 * 16) * 4));
@@ -1925,7 +1928,10 @@ bool prefill_sums_splits(int candidate, int K, int64_t tokens, int ks) {
 }
 
 bool prefill_partials_pay(int candidate, int M, int K, int64_t tokens, int ks, int cus) {
-  if (!prefill_sums_splits(candidate, K, tokens, ks)) return true;
+  // Partials of more than a dozen splits are summed faster by the reduce kernel than by a consumer, its launch
+  // included: 2048 x 11008 at 77 tokens (16 splits) 22.4 against 23.2 us and at 128 26.2 against 28.2, 5120 x 27648 at
+  // 20 (25) 37.3 against 40.7; 2560 x 9728 at 112 (12) 25.8 against 25.5.
+  if (!prefill_sums_splits(candidate, K, tokens, ks)) return ks <= 12;
   // With a consumer that reads the partials (no reduce launch) against the split-group tile and the plain consumer: the
   // tile is faster up to 64 tokens (4096 x 4096 at 20 14.9 / 11.8 us, 12288 x 5120 at 64 30.6 / 31.6) and in one round
   // of the CUs (8192 x 3072 at 96 23.4 / 17.9); in two the partials are (7168 x 5120 at 97 26.7 / 30.2 and at 128

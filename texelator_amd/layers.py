@@ -345,8 +345,7 @@ def linear_swiglu_prefill(handle: int, x: torch.Tensor, out: torch.Tensor | None
 
 def prefill_plan(handle: int, tokens: int) -> int:
     """The faster path for a call of ``tokens`` tokens (``_lib.TX_PREFILL_*``): K whole (``linear``), partials
-    (:func:`prefill_split` and a consumer), or split and summed in the tile (:func:`linear_into` and the plain
-    helper)."""
+    (:func:`prefill_split` and a consumer), or split and summed (:func:`linear_into` and the plain helper)."""
     out = ctypes.c_int(0)
     check(_lib.load().tx_prefill_plan(handle, int(tokens), out))
     return out.value
@@ -356,14 +355,17 @@ def linear_into(handle: int, x: torch.Tensor, out: torch.Tensor, workspace: torc
     """``linear(handle, x)`` of a bf16 x [tokens, K] into ``out`` [tokens, M], with a workspace of
     ``workspace_bytes(handle, tokens)`` bytes the caller keeps between calls on one stream."""
     m, k = _hip_shape(handle)
+    x_ptr, workspace_ptr = x.data_ptr(), workspace.data_ptr()
     _expect(x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and x.dim() == 2 and x.shape[1] == k
-            and x.data_ptr() % 16 == 0, "x must be a contiguous, 16-byte aligned CUDA bf16 [tokens, K] tensor")
-    _expect(out.dtype == torch.bfloat16 and out.is_contiguous() and out.shape == (x.shape[0], m) and out.device == x.device,
-            "out must be a contiguous bf16 [tokens, M] on x's device")
-    _expect(workspace.is_cuda and workspace.is_contiguous() and workspace.data_ptr() % 16 == 0,
+            and x_ptr % 16 == 0, "x must be a contiguous, 16-byte aligned CUDA bf16 [tokens, K] tensor")
+    tokens = x.shape[0]
+    _expect(out.is_cuda and out.dtype == torch.bfloat16 and out.is_contiguous() and out.shape == (tokens, m),
+            "out must be a contiguous CUDA bf16 [tokens, M]")
+    _expect(workspace.is_cuda and workspace.is_contiguous() and workspace_ptr % 16 == 0,
             "workspace must be a contiguous, 16-byte aligned CUDA tensor")
-    check(_lib.load().tx_linear(handle, _ptr(x), _lib.TX_DTYPE_BF16, x.numel(), k, x.device.index, _ptr(out), _ptr(workspace),
-                                workspace.numel() * workspace.element_size(), _stream(x)))
+    device = x.device
+    check(_lib.load().tx_linear(handle, x_ptr, _lib.TX_DTYPE_BF16, tokens * k, k, device.index, out.data_ptr(), workspace_ptr,
+                                workspace.nbytes, _stream_address(device)))
     return out
 
 
