@@ -143,7 +143,7 @@ class _Layer:
 
 
 class _SplitLinear(NamedTuple):
-    """A linear whose prefill GEMM splits K: the workspace of its partials and, where the tile sums them, its output."""
+    """A linear whose prefill GEMM splits K: the workspace of its partials and, where it sums them, its output."""
 
     workspace: torch.Tensor
     out: torch.Tensor | None
@@ -418,6 +418,8 @@ class BC4Decoder:
         prompt = (tokens > 1 and length == tokens and positions.data_ptr() == self.key_positions.data_ptr()
                   and self.flash_prompt_attention)
         split = self._split_linears(tokens)
+        epilogue = (tokens > 1 and self.gate_up_swiglu_prefill
+                    and layers.prefill_plan(self.layers[0].handles["gate_up"], tokens) == TX_PREFILL_WHOLE)
         for index, layer in enumerate(self.layers):
             qkv = self._prefill_linear(layer, "qkv", x, split.get("qkv"))
             if qkv is None:
@@ -435,15 +437,15 @@ class BC4Decoder:
             else:
                 attn = self._cached_attention(index, q.view(tokens, c.heads, c.head_dim), positions, length)
             self._add_rmsnorm_tokens(h, layer, "o", attn, layer.post_norm, x, split.get("o"))
-            act = self._gate_up_swiglu_tokens(layer, x)
+            act = self._gate_up_swiglu_tokens(layer, x, epilogue)
             following = self.layers[index + 1].input_norm if index + 1 < len(self.layers) else self.final_norm
             self._add_rmsnorm_tokens(h, layer, "down", act, following, x, split.get("down"))
         return x
 
     def _split_linears(self, tokens: int) -> dict[str, _SplitLinear]:
         """The linears (``qkv``, ``o``, ``down``) whose prefill GEMM of ``tokens`` tokens splits K, as the first
-        layer's handles plan it, with one workspace (every consumer runs before the next GEMM). Where the tile sums
-        its splits the plain consumer reads the linear's output: 13.1 against 16.4 us with partials for the 27B-class
+        layer's handles plan it, with one workspace (every consumer runs before the next GEMM). Where the splits are
+        summed faster by the linear the plain consumer reads its output: 13.1 against 16.4 us with partials for the 27B-class
         q|k|v at 20 tokens, 21.0 against 23.5 for its o at 77, 10.1 against 16.0 for the 3B-class o at 128."""
         if not self.split_prefill or tokens < 2:
             return {}
@@ -545,11 +547,11 @@ class BC4Decoder:
             return layers.linear_swiglu(handle, x, out=self.act_buffer)
         return layers.swiglu(layer.linears["gate_up"](x))
 
-    def _gate_up_swiglu_tokens(self, layer: _Layer, x: torch.Tensor) -> torch.Tensor:
-        """SwiGLU of the merged gate|up projection of several tokens: one prefill GEMM with the
-        SwiGLU epilogue where the call's tile supports it unsplit (bit-identical to the GEMM +
+    def _gate_up_swiglu_tokens(self, layer: _Layer, x: torch.Tensor, epilogue: bool) -> torch.Tensor:
+        """SwiGLU of the merged gate|up projection of several tokens: with ``epilogue`` (the call may run unsplit) one
+        prefill GEMM with the SwiGLU epilogue where the call's tile supports it (bit-identical to the GEMM +
         SwiGLU kernels it replaces), else those two kernels."""
-        if x.shape[0] > 1 and self.gate_up_swiglu_prefill:
+        if epilogue:
             try:
                 return layers.linear_swiglu_prefill(layer.handles["gate_up"], x)
             except UnsupportedError:
