@@ -108,16 +108,17 @@ hipError_t launch_gemv_swiglu(const GemvParams &p, int lookahead, hipStream_t st
 constexpr int kPrefillFirst = 5;
 constexpr int kPrefillLast = 9;
 bool prefill_candidate_eligible(int candidate, int M, int K);
-// K splits of the prefill GEMM for a shape (the same for every candidate).
-// Default tile by shape (the autotuner's profile overrides it): measured best on the 27B-class
-// shapes -- small_32x128 up to 32 tokens, and up to 128 where its split-group form pays (prefill.hip),
-// else medium_64x128 up to 64, medium_128x128 below 256 (two
-// workgroups per CU, which hide each other's LDS and decode latency), from 256 tokens
-// large_256x128 (decode shared by wave pairs) when its workgroups make one round of the CUs at
-// least three quarters full. prefill_register_candidate: the same without the split-group form, for
-// callers that want the splits' partials (tx_prefill_split).
+// Default tile by shape (the autotuner's profile overrides it), measured best on the 27B-class shapes and generic ones:
+// small_32x128 up to 32 tokens, and up to 128 where its split-group form pays (prefill.hip), else
+// medium_64x128 up to 64, medium_128x128 below 256 (two workgroups per CU, which hide each other's
+// LDS and decode latency); from 384 tokens the wide tile where at most a quarter of its last 512 tokens is
+// padding and its workgroups fill the rounds of the CUs they make; else from 256 tokens medium_128x128 where the
+// last 256 tokens are at most half full, and large_256x128 (decode shared by wave pairs) when its
+// workgroups make one round of the CUs at least three quarters full. prefill_register_candidate: the
+// same without the split-group form, for callers that want the splits' partials (tx_prefill_split).
 int prefill_default_candidate(int M, int K, int64_t tokens, int cus);
 int prefill_register_candidate(int M, int K, int64_t tokens, int cus);
+// K splits of the prefill GEMM for a shape (the same for every candidate).
 int prefill_splits(int M, int K, int64_t tokens, int cus);
 // Whether a call of `tokens` tokens with `ks` splits sums them inside the tile `candidate` (the split-group form: no
 // partials, no reduce launch) unless its partials are asked for.

@@ -1881,14 +1881,12 @@ int prefill_register_candidate(int M, int K, int64_t tokens, int cus) {
   // finer grain fills sparse grids and the last of several rounds better.
   const int64_t items = (int64_t)((M + 127) / 128) * ((tokens + 255) / 256);
   if (items > (int64_t)cus) return 6;
-  // Where the last 256 tokens are at most half full, the 128x128 tile (two workgroups a CU) has less padding, if
-  // its workgroups make at least one and a quarter rounds of the CUs. Before and now, with the wide tile's
-  // three-quarters rule above: 5120 x 5120 at 320 tokens 46.7 -> 42.3 us, 5120 x 27648 154.7 -> 132.1, 13824 x 5120
-  // 85.5 -> 81.5; at 520 tokens 4096 x 4096 58.3 -> 40.5, 27648 x 5120 269.1 -> 211.4. Below the line 3000 x 4848
-  // at 333 tokens in fp16 (288 workgroups) 33.2 us, 33.7 on the 128x128 tile.
-  const int64_t fine = (int64_t)((M + 127) / 128) * ((tokens + 127) / 128);
-  const int64_t fine_ks = std::min<int64_t>(std::max<int64_t>(1, 2 * (int64_t)cus / fine), std::max(1, CG / 8));
-  if ((tokens - 1) % 256 < 128 && 4 * fine * fine_ks >= 5 * (int64_t)cus) return 6;
+  // Where the last 256 tokens are at most half full, the 128x128 tile (two workgroups a CU) has less padding. Before and
+  // now, with the wide tile's three-quarters rule above: 5120 x 5120 at 320 tokens 46.7 -> 42.3 us, 5120 x 27648 154.7
+  // -> 132.1, 13824 x 5120 85.5 -> 81.5; at 520 tokens 4096 x 4096 58.3 -> 40.5, 27648 x 5120 269.1 -> 211.4. Least where
+  // its workgroups make 1.125 rounds of the CUs (here they make no fewer): ten shapes of 1536 to 12288 rows at 257
+  // to 384 tokens in both types 2.8% slower (6144 x 2048) to 4% faster (12288 x 8192), level on average.
+  if ((tokens - 1) % 256 < 128) return 6;
   return 4 * items * splits(items) >= 3 * (int64_t)cus ? 5 : 6;
 }
 
