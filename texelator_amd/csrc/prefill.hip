@@ -1584,49 +1584,43 @@ __global__ __launch_bounds__(kWideThreads) void prefill_wide_kernel(PrefillParam
 // KS > 0: exactly KS splits, every partial loaded before the first add; KS = 0: any count, eight loads
 // at a time (a loop over single loads waited for memory once per split: 5 to 25 splits are usual).
 constexpr int kReduceMaxKS = 16;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 template <bool F16, int KS>
 __global__ __launch_bounds__(256) void prefill_reduce_kernel(PrefillParams p) {
-  const int m = (blockIdx.x * 256 + threadIdx.x) * 4;
+  const int m = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
   const int t = blockIdx.y;
   if (m >= p.M) return;
-  const float4 *src = reinterpret_cast<const float4 *>(p.partials + (size_t)t * p.Mp + m);  // Mp is a multiple of 16
+  const f32x4 *src = reinterpret_cast<const f32x4 *>(p.partials + (size_t)t * p.Mp + m);  // Mp is a multiple of 16
   const size_t stride = (size_t)p.tokens * p.Mp / 4;
-  float4 total = make_float4(0.f, 0.f, 0.f, 0.f);
-  auto add = [&](const float4 &v) {
-    total.x += v.x;
-    total.y += v.y;
-    total.z += v.z;
-    total.w += v.w;
-  };
+  f32x4 total = {0.f, 0.f, 0.f, 0.f};
   uint16_t b[4] = {0, 0, 0, 0};
   if (p.bias) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) b[e] = static_cast<const uint16_t *>(p.bias)[min(m + e, p.M - 1)];
   }
   if constexpr (KS > 0) {
-    float4 v[KS];
+    f32x4 v[KS];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) v[s] = src[s * stride];
+    for (int s = 0; s < KS; ++s) v[s] = __builtin_nontemporal_load(src + s * stride);
     __builtin_amdgcn_sched_barrier(0);  // every load issued before the first add
 #pragma unroll
-    for (int s = 0; s < KS; ++s) add(v[s]);
+    for (int s = 0; s < KS; ++s) total += v[s];
   } else {
     constexpr int kGroup = 8;
     for (int s0 = 0; s0 < p.ks; s0 += kGroup) {
-      float4 v[kGroup];
+      f32x4 v[kGroup];
 #pragma unroll
-      for (int u = 0; u < kGroup; ++u) v[u] = src[(size_t)min(s0 + u, p.ks - 1) * stride];
+      for (int u = 0; u < kGroup; ++u) v[u] = __builtin_nontemporal_load(src + (size_t)min(s0 + u, p.ks - 1) * stride);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int u = 0; u < kGroup; ++u)
-        if (s0 + u < p.ks) add(v[u]);
+        if (s0 + u < p.ks) total += v[u];
     }
   }
-  const float sums[4] = {total.x, total.y, total.z, total.w};
   uint16_t out[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    float v = round_out<F16>(sums[e]);
+    float v = round_out<F16>(total[e]);
     if (p.bias) v += half_bits_to_float<F16>(b[e]);
     out[e] = F16 ? __builtin_bit_cast(uint16_t, (_Float16)v) : to_bf(v);
   }
@@ -1652,12 +1646,18 @@ struct Candidate {
 // The ordered reduction of the split-K partials, after the tile kernel.
 template <bool F16, int KS = 2>
 void launch_reduce_as(const PrefillParams &p, hipStream_t stream) {
-  const dim3 grid((p.M + 1023) / 1024, p.tokens);
+  // Columns of a workgroup: 1024 up to 4096 rows, else 256. The kernel itself is level (16384 x 4096 at 128 tokens
+  // 6.8 / 7.1 us), but the width decides which XCDs hold the partials' lines when the next tile kernel writes them:
+  // with 1024 that call's tile took 35.8 us instead of 31.5 (call by call 41.8 / 39.6, 8192 x 13824 at 97 tokens
+  // 52.6 / 50.3), with 256 a 2048 x 11008 call at 255 tokens 34.8 us instead of 31.8. Non-temporal loads, as the
+  // partials are read once: 2 to 3% of the call (2048 x 11008 at 97 21.8 -> 21.1, 8192 x 4848 at 97 26.7 -> 26.1).
+  const int threads = p.M <= 4096 ? 256 : 64;
+  const dim3 grid((p.M + 4 * threads - 1) / (4 * threads), p.tokens);
   if constexpr (KS <= kReduceMaxKS) {
-    if (p.ks == KS) hipLaunchKernelGGL((prefill_reduce_kernel<F16, KS>), grid, dim3(256), 0, stream, p);
+    if (p.ks == KS) hipLaunchKernelGGL((prefill_reduce_kernel<F16, KS>), grid, dim3(threads), 0, stream, p);
     else launch_reduce_as<F16, KS + 1>(p, stream);
   } else {
-    hipLaunchKernelGGL((prefill_reduce_kernel<F16, 0>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((prefill_reduce_kernel<F16, 0>), grid, dim3(threads), 0, stream, p);
   }
 }
 
