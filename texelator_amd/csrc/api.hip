@@ -189,6 +189,7 @@ int run_prefill(Handle *h, int candidate, const void *x, bool f16, int64_t token
                 int64_t workspace_bytes, hipStream_t stream) {
   if (candidate == kDenseBackend) return run_dense_prefill(h, x, f16, tokens, y, workspace, workspace_bytes, stream);
   tx::PrefillParams p{};
+  p.cus = h->cus;
   p.f16 = f16 ? 1 : 0;
   p.lut = h->lut;
   p.tiles = h->tiles;
@@ -956,6 +957,7 @@ int tx_linear_swiglu_prefill(uint64_t value, const void *x, int64_t tokens, void
                                     "backend, or splits K (use tx_linear + tx_swiglu)");
   DeviceGuard guard(h->device);
   tx::PrefillParams p{};
+  p.cus = h->cus;
   p.lut = h->lut;
   p.tiles = h->tiles;
   p.scales = h->scales;
@@ -1015,6 +1017,7 @@ int tx_prefill_split(uint64_t value, const void *x, int64_t tokens, void *worksp
     return fail(TX_ERR_INVALID, "prefill_split: workspace missing or too small (see tx_workspace_bytes)");
   DeviceGuard guard(h->device);
   tx::PrefillParams p{};
+  p.cus = h->cus;
   p.lut = h->lut;
   p.tiles = h->tiles;
   p.scales = h->scales;

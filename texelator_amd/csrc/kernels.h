@@ -84,6 +84,7 @@ struct PrefillParams {
   void *y;                 // [tokens][M] bf16
   float *partials;         // [ks][tokens][Mp] when ks > 1 (caller's workspace)
   int M, K, Mp, RG, CG, tokens, ks;
+  int cus;                 // of the device
   int f16;                 // x, bias and y are fp16 (weights rounded to fp16) instead of bf16
   const float4 *lut;       // LUT mode: 255 x 255 x 8 fp32 palette table, or nullptr (defined palette)
   int no_reduce;           // with ks > 1: leave the partials for a consumer (no reduce kernel)

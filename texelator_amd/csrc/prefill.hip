@@ -1748,7 +1748,6 @@ int wave_token_blocks(int row_blocks, int token_tiles, int cus) {
   return token_tiles == 1 ? 1 : 2;
 }
 
-constexpr int kWaveCus = 256;           // MI355X
 constexpr int kWaveMaxTokens = 128;     // four token tiles
 constexpr int kWaveMinColumns = 16, kWaveMaxColumns = 64;  // K tiles of 128
 
@@ -1778,7 +1777,7 @@ void launch_wave_as(const PrefillParams &p, hipStream_t stream) {
   // workgroups, 35.9 us; four, 216 workgroups, 31.5 us).
   const int row_blocks = (p.M + 31) / 32, token_tiles = (p.tokens + 31) / 32;
   const int wide = (row_blocks + 1) / 2 * token_tiles;
-  const int tbw = wave_token_blocks(row_blocks, token_tiles, kWaveCus);
+  const int tbw = wave_token_blocks(row_blocks, token_tiles, p.cus);
   const bool two_rows = token_tiles == 1 && wide >= TX_WAVE_RBW2_MIN_WGS;
   const int wgs = two_rows ? wide : row_blocks * ((token_tiles + tbw - 1) / tbw);
   const dim3 grid((wgs + kXcds - 1) / kXcds * kXcds), threads(kThreads);
