@@ -10,7 +10,7 @@
 // about 1500 launches, each a pass over [blocks][16] arrays in memory. Here the weights are read once
 // from HBM (the second read of a row hits the caches) and only the blocks are written. What is left
 // is VALU work: nine candidate palettes of eight values against sixteen weights, ~4000 instructions a
-// block; 174 us for that matrix, its issue floor being ~165. Five waves per SIMD (96 registers, 124 bytes
+// block; 174 us for that matrix, launches back to back (194 the best of ten in a trace), its issue floor being ~165. Five waves per SIMD (96 registers, 120 bytes
 // spilled in the least squares) hide the palette gathers better than three without spills (238 us).
 #include "bc4_device.h"
 #include "kernels.h"
@@ -146,9 +146,7 @@ __device__ __forceinline__ uint2 encode_one(const float (&v)[16], const float (&
 
   // 3. the 3 x 3 neighbourhood: weighted squared error, the first strict improvement wins. Only
   // the distance to the nearest value is needed here; the selectors are found once, at the end.
-  // A block that holds a NaN (hi is one) keeps its start, as every torch error of it is NaN: the minima
-  // below skip NaN, and negative importances would turn what they leave into an improvement.
-  float best_error = hi != hi ? -INFINITY : INFINITY;
+  float best_error = INFINITY;
 #pragma unroll 1
   for (int d0 = -1; d0 <= 1; ++d0) {
     const int c0 = min(max(center0 + d0, -127), 127);
@@ -207,6 +205,15 @@ __global__ __launch_bounds__(kEncodeMaxThreads, 5) void encode_rows_kernel(const
     load16<kF32>(hdiag, (size_t)b * 16, h);
 #pragma unroll
     for (int i = 0; i < 16; ++i) v[i] = clamp_nan(v[i] / scale, -1.f, 1.f);
+    // A block that holds a NaN keeps its start, as every torch error of it is NaN. The search's minima skip NaN,
+    // and negative importances would turn the infinity they leave into an improvement: positive ones never do.
+    if (!(scale < INFINITY)) {  // NaN or infinite weights in the row: the same for the workgroup
+      bool nan = false;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) nan |= v[i] != v[i];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) h[i] = nan ? 1.f : h[i];
+    }
     blocks[row * nblk + b] = encode_one(v, h, lut, coefficients);
   }
 }
