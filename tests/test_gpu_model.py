@@ -415,7 +415,7 @@ def test_decoder_prefill_with_split_consumers_is_bit_identical(ext, config):
         model.close()
 
 
-@pytest.mark.parametrize("tokens,split", [(20, set()), (77, set()), (128, set()), (200, {"qkv", "o", "down"})])
+@pytest.mark.parametrize("tokens,split", [(20, set()), (77, set()), (128, {"down"}), (200, {"qkv", "o", "down"})])
 def test_short_prompts_take_the_faster_path(ext, monkeypatch, tokens, split):
     """A 3B-class layer: where linear's default is the split-group tile (q|k|v and o up to 128 tokens), or more than a
     dozen splits are reduced (down), the prompt takes the linear, elsewhere the partials go to the consumer; the hidden

@@ -74,10 +74,12 @@ def test_k_that_was_whole_stays_whole(ext):
 
 
 @pytest.mark.parametrize("m,k,tokens,ks", [(3000, 4848, 128, 9), (3000, 4848, 129, 4), (1536, 8960, 200, 8),
-                                           (2560, 2048, 200, 4), (2048, 11008, 128, 16), (2048, 11008, 129, 10),
+                                           (2560, 2048, 200, 4), (2048, 11008, 127, 16), (2048, 11008, 128, 10),
+                                           (4096, 4848, 127, 8), (4096, 4848, 128, 4),
                                            (1024, 4096, 32, 4), (960, 4096, 33, 8), (256, 4992, 17, 4), (1024, 4112, 32, 8)])
 def test_finer_splits_only_where_they_pay(ext, m, k, tokens, ks):
-    """Past 128 tokens where they at least double the splits; up to 32 not where the split-group tile runs."""
+    """Past 128 tokens where they at least double the splits; below 16 MiB of partials; up to 32 tokens not where the
+    split-group tile runs."""
     handle = pack(ext, m, k, "bf16")[0]
     try:
         assert splits(ext, handle, m, tokens) == ks

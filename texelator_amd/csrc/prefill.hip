@@ -1907,13 +1907,17 @@ int prefill_splits(int M, int K, int64_t tokens, int cus) {
   // 1536 x 8960 at 255 26.7 with eight, 27.4 with ten. A K that was not split stays whole.
   int64_t fine = tokens < 256 && coarse > 1 ? std::min<int64_t>(CG / 4, cus / items) : 1;
   if (tokens > 128 && fine < 2 * coarse) fine = 1;
+  // Nor where the finer splits' partials reach 16 MiB: 4096 x 4848 at 128 tokens 23.1 us with eight
+  // splits, 22.3 with four, 2048 x 11008 23.3 with sixteen, 22.9 with ten (at 120 tokens, 15 MiB, the finer are level
+  // or faster).
+  const int64_t split_bytes = tokens * (int64_t)((M + 15) / 16 * 16) * 4;
+  if (fine * split_bytes >= int64_t(16) << 20) fine = 1;
   // Nor where four splits run the split-group tile (up to 32 tokens), which needs no reduce launch: 1024 x 4096 at 17
   // tokens 8.8 us against 9.5 with eight, 256 x 4096 8.5 / 9.1, 512 x 4608 9.2 / 9.3.
   if (prefill_sums_splits(dc, K, tokens, (int)std::min(ks, coarse))) fine = 1;
   ks = std::min(ks, std::max(coarse, fine));
   if (ks > 1 && wave_tile_pays(M, K, tokens, cus)) ks = 4;
-  const int64_t cap = std::max<int64_t>(1, (int64_t(32) << 20) / (tokens * (int64_t)((M + 15) / 16 * 16) * 4));
-  ks = std::min(ks, cap);
+  ks = std::min(ks, std::max<int64_t>(1, (int64_t(32) << 20) / split_bytes));
   ks = std::min<int64_t>(ks, std::max(1, 0x7FFFFFFF / std::max(CG, 1)));  // the kernels' 32-bit split arithmetic
   return (int)std::max<int64_t>(1, ks);
 }
@@ -1929,7 +1933,7 @@ bool prefill_sums_splits(int candidate, int K, int64_t tokens, int ks) {
 
 bool prefill_partials_pay(int candidate, int M, int K, int64_t tokens, int ks, int cus) {
   // Partials of more than a dozen splits are summed faster by the reduce kernel than by a consumer, its launch
-  // included: 2048 x 11008 at 77 tokens (16 splits) 22.4 against 23.2 us and at 128 26.2 against 28.2, 5120 x 27648 at
+  // included: 2048 x 11008 at 77 tokens (16 splits) 22.4 against 23.2 us and at 112 24.6 against 26.1, 5120 x 27648 at
   // 20 (25) 37.3 against 40.7; 2560 x 9728 at 112 (12) 25.8 against 25.5.
   if (!prefill_sums_splits(candidate, K, tokens, ks)) return ks <= 12;
   // With a consumer that reads the partials (no reduce launch) against the split-group tile and the plain consumer: the
