@@ -10,8 +10,9 @@
 // about 1500 launches, each a pass over [blocks][16] arrays in memory. Here the weights are read once
 // from HBM (the second read of a row hits the caches) and only the blocks are written. What is left
 // is VALU work: nine candidate palettes of eight values against sixteen weights, ~4000 instructions a
-// block; 174 us for that matrix, launches back to back (194 the best of ten in a trace), its issue floor being ~165. Five waves per SIMD (96 registers, 120 bytes
-// spilled in the least squares) hide the palette gathers better than three without spills (238 us).
+// block; 174 us for that matrix, launches back to back (the best of ten cold ones in a trace 191), its issue floor
+// being ~165. Five waves per SIMD (96 registers, 120 bytes spilled in the least squares) hide the palette gathers
+// better than three without spills (238 us).
 #include "bc4_device.h"
 #include "kernels.h"
 

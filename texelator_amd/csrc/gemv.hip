@@ -316,7 +316,8 @@ __device__ __forceinline__ void tile_mfma(uint4 cur, const XFrag &xf, float scal
 // and 2j + 1 load one row together, half a row each, first the even lane's row, then the odd lane's (32
 // lines an instruction, the same number of instructions), and exchange halves by DPP when they are used.
 // Measured with both forms: 17408 x 5120 at 1 token 43.8 -> 37.1 us and at 8 tokens 52.7 -> 42.8, 27648 x 5120
-// 64.5 -> 51.0, 5120 x 5120 16.7 -> 14.8, fp16 2048 x 11008 at 4 tokens 23.9 -> 17.5, 256 x 2048 4.8 both.
+// 64.5 -> 51.0, 5120 x 5120 16.7 -> 14.8, fp16 2048 x 11008 at 4 tokens 23.9 -> 17.5, 256 x 2048 4.8 both. A grid of one
+// to eight row groups at 2 to 4 tokens, bound by latency, is level to 14% slower (16 x 5120 at 2 tokens 6.6 -> 7.7).
 struct TileRows {
   float4 a_even, a_odd, b_even, b_odd;  // this lane's half (its parity) of the pair's rows, blocks a and b
 };
