@@ -1,7 +1,7 @@
 """Throughput of the gfx950 BC4 decode GEMV on the 27B-class linear shapes (batch 1).
 
 One "step" is one decode sweep: every q, k, v, o, gate, up and down linear of ``--layers``
-distinct layer copies, each a batch-1 GEMV with a float32 output (BASELINE config 2). The
+distinct layer copies, each a batch-1 GEMV with a float32 output. The
 copies are distinct device buffers, together far larger than the 256 MB Infinity Cache, so the
 weights stream from HBM. A step is captured once as a HIP graph and replayed.
 
@@ -14,11 +14,11 @@ decode + matvec, of the decode and of the matvec alone, and the config-3 fp32 GE
 ``hbm_stream_read`` is a plain streaming read of the same launch size (the achievable HBM rate);
 ``roofline.frac_of_stream_read`` is the GEMV's rate against it.
 ``prefill_tok_s_512`` and ``decode_tok_s`` are the metric's other two figures on the 27B-class
-decoder (linears BC4-encoded from random-init weights): the 512-token prefill
+decoder (64 layers, hidden 5120, linears BC4-encoded from random-init weights): the 512-token prefill
 (``texelator_amd.prefill.benchmark_prefill``; null with ``prefill_gate_failed`` if the prefill path
 fails the reference protocol's correctness gate) and graph-replayed greedy decode from 512 to
-``--context`` with every step timed; ``model`` holds the details, ``model_3b`` the same for BASELINE
-config 4, and ``model_3b_hf`` config 4 through the reference's own calling path (a Hugging Face
+``--context`` with every step timed; ``model`` holds the details, ``model_3b`` the same for the
+3B-class one, and ``model_3b_hf`` that one through the reference's own calling path (a Hugging Face
 Qwen2 with TexelatorLinear modules: prefill protocol and greedy ``generate``).
 """
 from __future__ import annotations
@@ -376,7 +376,7 @@ def fp4_only(torch, ext, runtime, hardware, device, args) -> int:
 def model_section(torch, args, model_name: str | None = None, context: int | None = None) -> dict:
     """Prefill tok/s at ``--prompt`` tokens (reference protocol, texelator/prefill.py:63-131) and
     graph-replayed greedy decode tok/s from the prompt up to ``context``, on a random-init BC4
-    decoder of BASELINE config 5 (27b) or 4 (3b) whose linears are BC4-encoded by this build's
+    decoder of the 27B class (27b) or the 3B class (3b) whose linears are BC4-encoded by this build's
     encoder (``--model-weights uniform``: uniform random block bytes instead). If the prefill path
     fails the protocol's correctness gate, the failure is reported and the prefill is not timed."""
     from texelator_amd import modeling, prefill
@@ -420,7 +420,7 @@ def model_section(torch, args, model_name: str | None = None, context: int | Non
 
 
 def hf_section(torch, args) -> dict:
-    """BASELINE config 4 through the reference's calling path: a Hugging Face Qwen2 with
+    """The 3B-class decoder through the reference's calling path: a Hugging Face Qwen2 with
     TexelatorLinear modules (``texelator_amd.hf.build_qwen2``), the reference's prefill protocol on
     it (``model.model(input_ids=...)``) and greedy ``model.generate`` of 256 tokens after a 512-token
     prompt, timed on the host clock (``hf.benchmark_generate``); then the same model decoding 256
@@ -486,15 +486,15 @@ def main() -> int:
     parser.add_argument("--no-graph", action="store_true", help="launch eagerly instead of replaying a graph")
     parser.add_argument("--no-prefill", action="store_true", help="skip the prefill GEMM measurements")
     parser.add_argument("--model", choices=("27b", "3b", "none"), default="27b",
-                        help="model-level decode/prefill tok/s on a random-init BASELINE config 5 (27b) or 4 (3b)")
+                        help="model-level decode/prefill tok/s on a random-init 27B- or 3B-class decoder")
     parser.add_argument("--context", type=int, default=4096, help="decode up to this context")
     parser.add_argument("--no-small-model", action="store_true",
-                        help="skip the Qwen2.5-3B-style decoder (BASELINE config 4) after the 27B-class one")
+                        help="skip the Qwen2.5-3B-style decoder after the 27B-class one")
     parser.add_argument("--prompt", type=int, default=512, help="prefill tokens")
     parser.add_argument("--model-weights", choices=("encoded", "uniform"), default="encoded",
                         help="BC4 data of the model-level decoders: encoded random-init weights or uniform bytes")
     parser.add_argument("--no-hf", action="store_true",
-                        help="skip the Hugging Face (reference calling path) measurement of BASELINE config 4")
+                        help="skip the Hugging Face (reference calling path) measurement of the 3B-class decoder")
     parser.add_argument("--hf-only", action="store_true",
                         help="run only the 3B model through Hugging Face modules (the model_3b_hf section)")
     parser.add_argument("--model-only", action="store_true",
@@ -675,14 +675,14 @@ def main() -> int:
         log(f"model-level tok/s ({args.model})")
         result["model"] = model_section(torch, args)
     if args.model == "27b" and not args.no_small_model:
-        # BASELINE config 4 as stated there: 512-token prompt, then 256 greedy decode steps
+        # the 3B-class decoder: 512-token prompt, then 256 greedy decode steps
         log("model-level tok/s (3b)")
         result["model_3b"] = model_section(torch, args, "3b", args.prompt + 256)
     if args.model != "none" and not args.no_hf:
         log("model-level tok/s (3b, Hugging Face calling path)")
         result["model_3b_hf"] = hf_section(torch, args)
     if "model" in result:
-        # the metric's second and third figures, fully timed; a prefill that
+        # the metric's second and third figures (27B-class decoder), fully timed; a prefill that
         # fails the reference protocol's correctness gate is reported as failed, not timed
         result["prefill_tok_s_512"] = result["model"]["prefill_tok_s"]
         result["prefill_gate_failed"] = result["model"]["prefill_gate_failed"]

@@ -51,6 +51,6 @@ def small_cases() -> dict[str, tuple[torch.Tensor, torch.Tensor, int]]:
 
 
 def config1_inputs() -> tuple[torch.Tensor, torch.Tensor]:
-    """BASELINE config 1: W 4096x4096 ~ N(0, 0.02^2) * LogNormal(0, 0.3) per input channel."""
+    """W 4096x4096 ~ N(0, 0.02^2) * LogNormal(0, 0.3) per input channel."""
     g = torch.Generator().manual_seed(20260827)
     return _lognormal_columns(4096, 4096, g), torch.ones(4096)

@@ -7,7 +7,7 @@ module name, so it cannot shadow this repository's package), runs it on the CPU 
 build's palette as the LUT, and stores inputs and outputs as data:
 
   tests/golden/encoder_vectors.npz   small cases: weight, hdiag, rows_per_chunk -> blocks, scales
-  tests/golden/encoder_vectors.json  BASELINE config 1 (4096 x 4096): SHA-256 of blocks and scales
+  tests/golden/encoder_vectors.json  the 4096 x 4096 matrix: SHA-256 of blocks and scales
 
 Run in the build container only (the reference does not exist on the GPU box):
     python tests/golden/make_encoder_vectors.py [/root/reference]
@@ -70,7 +70,7 @@ def main() -> None:
     weight, hdiag = config1_inputs()
     blocks, scales = encode(encoder, weight, hdiag, lut, 128)
     record = {
-        "case": "BASELINE config 1: W 4096x4096 ~ N(0, 0.02^2) * LogNormal(0, 0.3) per input channel, "
+        "case": "W 4096x4096 ~ N(0, 0.02^2) * LogNormal(0, 0.3) per input channel, "
                 "seed 20260827, hdiag = 1, rows_per_chunk 128",
         "torch": torch.__version__,
         "palette_sha256": bc4.palette_sha256(),

@@ -36,7 +36,7 @@ def bf16_bits(t: torch.Tensor) -> np.ndarray:
 
 
 def config_weight(m: int, k: int, seed: int) -> torch.Tensor:
-    """``W ~ N(0, 0.02^2)`` scaled per input channel by ``LogNormal(0, 0.3)`` (BASELINE configs 1-3)."""
+    """``W ~ N(0, 0.02^2)`` scaled per input channel by ``LogNormal(0, 0.3)``."""
     generator = torch.Generator().manual_seed(seed)
     w = torch.randn((m, k), generator=generator) * 0.02
     s = torch.exp(0.3 * torch.randn(k, generator=generator))

@@ -105,7 +105,7 @@ def test_hf_generate_greedy(qwen_pair):
 
 
 def test_calibrated_artifact_installed_standalone_matches_dense(ext, tmp_path):
-    """BASELINE-style offline pipeline (reference: converter.py:62-233, runtime.py:242-263,
+    """The offline pipeline (reference: converter.py:62-233, runtime.py:242-263,
     standalone.py:102-158): E[x^2] moments from a local token file drive the GPU encoder into a
     resumable artifact; ``install_standalone`` puts its handles into a meta-initialised Qwen2
     whose remaining tensors are then assigned (as the standalone loader does); its logits match
@@ -159,7 +159,7 @@ def test_calibrated_artifact_installed_standalone_matches_dense(ext, tmp_path):
 
 
 def test_build_qwen2_reference_prefill_protocol_and_generate(ext):
-    """The reference's calling path at BASELINE config-4 shapes (4 of its 36 layers, so the test
+    """The reference's calling path at the 3B-class shapes (4 of its 36 layers, so the test
     stays short): ``hf.build_qwen2`` puts TexelatorLinear modules holding GPU-encoded random-init
     weights into a meta-initialised Qwen2, ``prefill.benchmark_prefill`` runs the reference's
     protocol on it (``model.model(input_ids=...)``, scalar-vs-hybrid gate on 32 tokens), and

@@ -1,6 +1,6 @@
 """GPU parity of the gfx950 BC4 path against the CPU oracle, through the C ABI.
 
-Bars (BASELINE north star): decoded weights bit-exact; GEMV fp32 output within 1e-3 relative
+Bars: decoded weights bit-exact; GEMV fp32 output within 1e-3 relative
 error of the float64 CPU matvec on the same decoded weights; prefill bf16 output within 1e-2
 relative RMS of the float64 CPU GEMM; all prefill candidates bitwise equal (the reference's
 autotuner gate, texelator/autotune.py:160-168).

@@ -1,11 +1,11 @@
-"""The reference's own calling path at a BASELINE model size: a Hugging Face Qwen2 whose seven
+"""The reference's own calling path at the size of a measured decoder: a Hugging Face Qwen2 whose seven
 linears per layer are :class:`~texelator_amd.runtime.TexelatorLinear` modules.
 
 The reference loads its standalone artifact into a meta-initialised Hugging Face model, puts
 ``TexelatorLinear`` modules in place of the linears (``standalone.py:102-158`` through
 ``runtime.install_standalone`` :242-263), assigns the remaining tensors, then decodes with
 ``model.generate`` (``cli._generate`` :189-219) and measures prefill with ``model.model(...)``
-(``prefill.py:24-26``). :func:`build_qwen2` does the same for a random-init BASELINE config 4 or 5
+(``prefill.py:24-26``). :func:`build_qwen2` does the same for a random-init 3B- or 27B-class
 model, its linears BC4-encoded on the GPU (or uniform blocks) with the same initialisation rules as
 :class:`~texelator_amd.modeling.BC4Decoder`; :func:`benchmark_generate` times greedy ``generate``.
 
@@ -33,7 +33,7 @@ LINEARS = ("self_attn.q_proj", "self_attn.k_proj", "self_attn.v_proj", "self_att
 
 
 def qwen2_config(config: DecoderConfig):
-    """The ``transformers.Qwen2Config`` of a BASELINE decoder config (untied lm_head, sdpa)."""
+    """The ``transformers.Qwen2Config`` of a decoder config (untied lm_head, sdpa)."""
     import transformers
 
     return transformers.Qwen2Config(

@@ -7,7 +7,7 @@ compact decoder with a static KV cache, so that a whole decode step (all layers,
 the cache update) can be captured once as a HIP graph and replayed per token. The host then
 does no per-token work, and decode speed is set by the GPU.
 
-Layer math follows Qwen2, the architecture of BASELINE configs 4 and 5:
+Layer math follows Qwen2, the architecture of the 3B- and 27B-class decoders:
 - RMSNorm in fp32 with ``weight * x``;
 - rotate-half RoPE with ``theta``;
 - grouped-query attention with q/k/v biases;
@@ -49,13 +49,13 @@ class DecoderConfig:
 
     @staticmethod
     def qwen25_3b_style() -> "DecoderConfig":
-        """BASELINE config 4."""
+        """The Qwen2.5-3B-style decoder: 36 layers, hidden 2048."""
         return DecoderConfig(layers=36, hidden=2048, heads=16, kv_heads=2, head_dim=128, intermediate=11008,
                              vocab=151936)
 
     @staticmethod
     def class_27b() -> "DecoderConfig":
-        """BASELINE config 5."""
+        """The 27B-class decoder: 64 layers, hidden 5120."""
         return DecoderConfig(layers=64, hidden=5120, heads=40, kv_heads=8, head_dim=128, intermediate=27648,
                              vocab=151936)
 
